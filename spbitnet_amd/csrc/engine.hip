@@ -1267,7 +1267,7 @@ __device__ __forceinline__ void split_weighted_v(const uint32_t (&vs)[kAttnSplit
 }
 
 // The per-split work of one query (the bs=1 and batched decode kernels share
-// it; the prefill kernel runs the same operations on register-held K and V):
+// it; the prefill kernel runs the same operations on the matrix cores):
 // once its q (qs, float) and the split's V rows (vs, bf16) are in
 // LDS behind a barrier and the thread holds its quarter of K row p = tid / 4
 // (kq; quarter tid % 4), the scores, the split's softmax and the weighted V
@@ -1487,170 +1487,285 @@ __global__ __launch_bounds__(kAttnThreads) void attention_kernel(
 
 // Prefill form: the queries of the tokens of a batch (token t at position
 // pos0 + t, its q at qkv + t * qkv_stride, its partials after those of
-// t - 1).  A block (split s, kv head, kQ consecutive tokens) loads the
-// split's K and V once and keeps both in registers for all of its tokens:
-//   * wave w holds quarter w of the head dims of K row j0 + lane, unpacked
-//     (kf), and reads each token's q quarters with scalar loads (the
-//     address is the same for the whole wave), so a score costs no LDS
-//     reads; the four quarter sums meet in LDS (red).
-//   * a V thread holds the element pair dp = tid % (HD/2) of all 64 rows of
-//     the split (vcol, bf16 pairs) and reads only the softmax weights from
-//     LDS.
-// The arithmetic is attention_split's, operation for operation, so a
-// prefilled token's partials equal those of its decode step:
+// t - 1), on the float32 matrix cores.  v_mfma_f32_16x16x4_f32 adds its four
+// products to the accumulator one after the other (k ascending), each as a
+// fused multiply-add rounded to nearest even, denormals kept: compared bit
+// for bit with fmaf on 21 M sums over normal, wide-exponent and denormal
+// operands.  So a chain of them is attention_split's fma chain, and every
+// partial equals that of the token's decode step:
 //   score = ((a0 + a1) + (a2 + a3)) * scale, a_w = fma chain over quarter w,
 //   the softmax of split_softmax, and acc = fma over j ascending of e_j v_j.
-template <int HD, int G, int kQ>
-__global__ __launch_bounds__(kAttnThreads) void attention_prefill_kernel(
+//
+// A block takes a kv head and an item: a split and some consecutive tokens
+// that reach it.  Its four waves put the split's K and V into LDS once, as float32 in operand
+// order (a lane's 16 bytes are the operands of four MFMAs), and then walk
+// over tiles of 16 rows (row = token, head of the group), each wave alone.
+//   * QK gives the transposed tile: A = K rows, B = q.  A's row i holds the
+//     tile's position 4 (i % 4) + i / 4, so accumulator v of lane (row n,
+//     group g) is the score of position 4 v + g, which is PV's A operand of
+//     step v without any exchange.
+//   * The dims of a step belong to the four lane groups in order; a lane
+//     loads 4 adjacent dims and the groups exchange them (transpose4).
+//   * PV's column n of tile e is dim (HD/16) n + e: 16-byte V loads, and a
+//     lane's results of a row are adjacent.
+// What bounds it: 256 MFMAs of 32 cycles per 16 rows x 64 positions (head_dim
+// 128) and ~575 VALU instructions, which do not overlap: float32 MFMAs and
+// VALU instructions of a SIMD's waves add up (15.2 ns per MFMA, ~1 ns more per
+// VALU instruction, measured).  Hence float32 operands in LDS: unpacking them
+// at each use took 256 more VALU instructions per tile (5.2 against 6.8 us for
+// a tile of a lone wave).  A 2048-token prompt's two passes of the 2B shape:
+// 197 + 375 us per layer with the VALU form this replaces, 74 + 171 us now
+// (5.3 us per tile and SIMD, 3.9 of it MFMA).
+__device__ __forceinline__ void swap16(float& a, float& b) {
+    const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(a), __float_as_uint(b), false,
+                                                    false);
+    a = __uint_as_float(r[0]);
+    b = __uint_as_float(r[1]);
+}
+__device__ __forceinline__ void swap32(float& a, float& b) {
+    const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(a), __float_as_uint(b), false,
+                                                    false);
+    a = __uint_as_float(r[0]);
+    b = __uint_as_float(r[1]);
+}
+// Register c of lane group g becomes register g of lane group c.
+__device__ __forceinline__ void transpose4(float (&r)[4]) {
+    swap16(r[0], r[1]);
+    swap16(r[2], r[3]);
+    swap32(r[0], r[2]);
+    swap32(r[1], r[3]);
+}
+// x: 4 registers whose lane groups hold adjacent positions.  The pairwise
+// tree's first two levels: lane group v gets (x_v g0 + g1) + (g2 + g3).
+__device__ __forceinline__ float quad_sums(float a, float b, float c, float d) {
+    swap16(a, b);
+    swap16(c, d);
+    float x = a + b, y = c + d;
+    swap32(x, y);
+    return x + y;
+}
+__device__ __forceinline__ void unpack_bf16x4(const uint2 x, float (&r)[4]) {
+    r[0] = __uint_as_float(x.x << 16);
+    r[1] = __uint_as_float(x.x & 0xFFFF0000u);
+    r[2] = __uint_as_float(x.y << 16);
+    r[3] = __uint_as_float(x.y & 0xFFFF0000u);
+}
+__device__ __forceinline__ bool bf16_pair_nonfinite(uint32_t w) {
+    return (w & 0x7F80u) == 0x7F80u || (w & 0x7F800000u) == 0x7F800000u;
+}
+
+typedef float v4f __attribute__((ext_vector_type(4)));
+
+struct PrefillItem {
+    int t0, n;   // tokens t0 .. t0 + n - 1 of the batch
+    int split;
+    int pos0;    // position of token t0
+    int jlast;   // last position of the batch's tokens
+    int pad;
+};
+template <int HD, int G>
+__global__ __launch_bounds__(kAttnThreads, HD == 128 ? 2 : 4) void attention_prefill_kernel(
     const uint16_t* __restrict__ qkv, const uint16_t* __restrict__ kc,
     const uint16_t* __restrict__ vc, float* __restrict__ pm, float* __restrict__ pl,
-    float* __restrict__ pacc, int max_seq, int S, float scale, int pos0, int nt,
-    int qkv_stride) {
-    constexpr int kU = HD / 8;
-    constexpr int kQU = kU / 4;       // 16-byte units per quarter row
-    constexpr int kQD = HD / 4;       // elements per quarter row
-    constexpr int kVP = HD / 2;       // element pairs per row
-    constexpr int kVRow = kVP + 1;
-    static_assert(kAttnThreads == 4 * kWave && kAttnSplit == kWave, "4 waves, lane = position");
-    static_assert(kAttnThreads % kVP == 0, "a thread's V pair is the same for all its heads");
-    __shared__ uint32_t vs[kAttnSplit][kVRow];
-    __shared__ float red[4][G][kAttnSplit];
-    __shared__ __align__(16) float sc[G][kAttnSplit];
-    __shared__ float hmax[G], hsum[G];
-    const int s = blockIdx.x, kvh = blockIdx.y;
+    float* __restrict__ pacc, int max_seq, int S, float scale, int nt, int qkv_stride,
+    const PrefillItem* __restrict__ items) {
+    constexpr int kTok = 16 / G;      // tokens per 16-row tile
+    constexpr int kM = HD / 16;       // 8-byte pieces of a row per lane; PV column tiles
+    constexpr int kQS = HD / 16;      // steps per quarter
+    constexpr int kVW = HD / 32;      // 32-bit V words per lane and row
+    constexpr int kWaves = kAttnThreads / kWave;
+    static_assert(kAttnSplit == 64 && kWaves == 4, "a wave fills one of four 16-position tiles");
+    typedef uint32_t vwords __attribute__((ext_vector_type(kVW)));
+    __shared__ v4f ks[4][kM][kWave];      // [tile][steps 4 m .. 4 m + 3][lane]
+    __shared__ v4f vs[16][kM / 4][kWave];  // [step][column tiles 4 u .. 4 u + 3][lane]
+    __shared__ int odd_v[kWaves];
+    const PrefillItem it = items[blockIdx.x];
+    const int s = it.split, kvh = blockIdx.y;
     const int j0 = s * kAttnSplit;
-    const int t0 = blockIdx.z * kQ;
-    const int t1 = t0 + kQ < nt ? t0 + kQ : nt;
-    if (j0 > pos0 + t1 - 1) return;  // no token of the block reaches the split
-    const int tid = threadIdx.x, lane = tid & (kWave - 1);
-    const int wq = __builtin_amdgcn_readfirstlane(tid / kWave);
+    const int t0 = it.t0, t1 = it.t0 + it.n;
+    const int pos0 = it.pos0 - it.t0;  // token t is at position pos0 + t
+    const int jlast = it.jlast;  // rows past it are not this prompt's
+    const int lane = threadIdx.x & (kWave - 1);
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+    const int n = lane & 15, g = lane >> 4;
     const long cache0 = static_cast<long>(kvh) * max_seq * HD;
-    const int jmax = max_seq - 1;
-    // quarter wq of K row j0 + lane (clamped to the cache) and the split's V
-    // rows (kVPer 16-byte units per thread), all loads issued together
-    uint4 kq[kQU];
+    // the wave's first tile with a token that reaches the split
+    constexpr int kStride = kWaves * kTok;
+    int tt = t0 + wave * kTok;
+    while (pos0 + tt + kTok - 1 < j0) tt += kStride;
+    auto load_q = [&](int tile, uint2 (&q)[kM]) {
+        const int t = tile + n / G < t1 ? tile + n / G : t1 - 1;
+        const uint2* qr = reinterpret_cast<const uint2*>(
+            qkv + static_cast<long>(t) * qkv_stride + (kvh * G + n % G) * HD);
+#pragma unroll
+        for (int m = 0; m < kM; ++m) q[m] = qr[4 * m + g];
+    };
+    uint2 qraw[kM];
     {
-        const int j = j0 + lane <= jmax ? j0 + lane : jmax;
-        const uint4* kr = reinterpret_cast<const uint4*>(kc + cache0 + static_cast<long>(j) * HD) +
-                          wq * kQU;
+        uint2 kraw[kM];
+        const int j = j0 + 16 * wave + 4 * (n & 3) + (n >> 2);
+        const uint2* kr = reinterpret_cast<const uint2*>(
+            kc + cache0 + static_cast<long>(j < jlast ? j : jlast) * HD);
 #pragma unroll
-        for (int u = 0; u < kQU; ++u) kq[u] = kr[u];
-    }
-    constexpr int kVPer = kAttnSplit * kU / kAttnThreads;
-    uint4 vraw[kVPer];
+        for (int m = 0; m < kM; ++m) kraw[m] = kr[4 * m + g];
+        vwords vraw[4];
 #pragma unroll
-    for (int i = 0; i < kVPer; ++i) {
-        const int idx = tid + i * kAttnThreads;
-        const int jj = idx / kU, c = idx - jj * kU;
-        const int j = j0 + jj <= jmax ? j0 + jj : jmax;
-        vraw[i] = reinterpret_cast<const uint4*>(vc + cache0 + static_cast<long>(j) * HD)[c];
-    }
+        for (int i = 0; i < 4; ++i) {
+            const int jv = j0 + 16 * wave + 4 * i + g;
+            vraw[i] = *reinterpret_cast<const vwords*>(
+                vc + cache0 + static_cast<long>(jv < jlast ? jv : jlast) * HD + kM * n);
+        }
+        load_q(tt, qraw);
 #pragma unroll
-    for (int i = 0; i < kVPer; ++i) {
-        const int idx = tid + i * kAttnThreads;
-        const int jj = idx / kU, c = idx - jj * kU;
-        uint32_t* row = &vs[jj][4 * c];
-        row[0] = vraw[i].x;
-        row[1] = vraw[i].y;
-        row[2] = vraw[i].z;
-        row[3] = vraw[i].w;
-    }
-    float kf[kQD];
+        for (int m = 0; m < kM; ++m) {
+            float r[4];
+            unpack_bf16x4(kraw[m], r);
+            transpose4(r);
+            ks[wave][m][lane] = (v4f){r[0], r[1], r[2], r[3]};
+        }
+        // A masked position's weight is 0; 0 * v drops out of the sum unless v
+        // is not finite.  Such a v in a split that some token sees only in
+        // part takes the path that skips masked positions.
+        bool odd = false;
 #pragma unroll
-    for (int u = 0; u < kQU; ++u) {
-        float f[8];
-        unpack_bf16x8(kq[u], f);
+        for (int i = 0; i < 4; ++i) {
 #pragma unroll
-        for (int e = 0; e < 8; ++e) kf[8 * u + e] = f[e];
+            for (int u = 0; u < kM / 4; ++u) {
+                float r[4];
+                unpack_bf16x4(make_uint2(vraw[i][2 * u], vraw[i][2 * u + 1]), r);
+                vs[4 * wave + i][u][lane] = (v4f){r[0], r[1], r[2], r[3]};
+            }
+#pragma unroll
+            for (int w = 0; w < kVW; ++w) odd |= bf16_pair_nonfinite(vraw[i][w]);
+        }
+        odd = __any(odd);
+        if (lane == 0) odd_v[wave] = odd;
     }
     __syncthreads();
-    const int dp = tid % kVP;
-    uint32_t vcol[kAttnSplit];
+    const bool odd = (odd_v[0] | odd_v[1] | odd_v[2] | odd_v[3]) != 0;
+    const unsigned hs = gridDim.y * G * S;
+    // the partials of the batch's nt tokens (alloc_prefill keeps them below 2 GB)
+    const __amdgpu_buffer_rsrc_t racc = __builtin_amdgcn_make_buffer_rsrc(
+        pacc, static_cast<short>(0), static_cast<int>(nt * hs * HD * 4), kBufferFlags);
+    const __amdgpu_buffer_rsrc_t rm = __builtin_amdgcn_make_buffer_rsrc(
+        pm, static_cast<short>(0), static_cast<int>(nt * hs * 4), kBufferFlags);
+    const __amdgpu_buffer_rsrc_t rl = __builtin_amdgcn_make_buffer_rsrc(
+        pl, static_cast<short>(0), static_cast<int>(nt * hs * 4), kBufferFlags);
+    constexpr unsigned kDropStore = 0xC0000000u;
+    for (; tt < t1; tt += kStride) {
+        asm volatile("" ::: "memory");  // K and V are read per tile: held in registers they would spill
+        float q[4 * kM];
 #pragma unroll
-    for (int jj = 0; jj < kAttnSplit; ++jj) vcol[jj] = vs[jj][dp];
-
-    // q element pairs of quarter wq of token t's heads (the address is the
-    // same for the whole wave: scalar loads); the next token's are loaded
-    // during the current token's softmax and V sums when they fit in SGPRs
-    constexpr int kQP = kQD / 2;
-    constexpr bool kPrefetchQ = G * kQP <= 64;
-    const uint32_t* q32 = reinterpret_cast<const uint32_t*>(qkv);
-    auto load_q = [&](int tt, uint32_t (&q)[G * kQP]) {
-        const uint32_t* qw =
-            q32 + (static_cast<long>(tt) * qkv_stride + (kvh * G) * HD + wq * kQD) / 2;
+        for (int m = 0; m < kM; ++m) {
+            float r[4];
+            unpack_bf16x4(qraw[m], r);
+            transpose4(r);
 #pragma unroll
-        for (int g = 0; g < G; ++g)
-#pragma unroll
-            for (int i = 0; i < kQP; ++i) q[g * kQP + i] = qw[g * kVP + i];
-    };
-    const long hs = static_cast<long>(gridDim.y) * G * S;
-    // the first token of the block that reaches the split
-    int t = t0;
-    if (j0 > pos0 + t) t = j0 - pos0;
-    uint32_t qn[G * kQP];
-    if (kPrefetchQ) load_q(t, qn);
-    for (; t < t1; ++t) {
-        const int pos = pos0 + t;
-        const int jn = (pos + 1 - j0) < kAttnSplit ? (pos + 1 - j0) : kAttnSplit;
-        // V stays packed (64 registers, not 128 unpacked ones): the block
-        // keeps 4 waves per SIMD
-#pragma unroll
-        for (int jj = 0; jj < kAttnSplit; ++jj) asm volatile("" : "+v"(vcol[jj]));
-        uint32_t qc[G * kQP];
-        if (kPrefetchQ) {
-#pragma unroll
-            for (int i = 0; i < G * kQP; ++i) qc[i] = qn[i];
-        } else {
-            load_q(t, qc);
+            for (int k = 0; k < 4; ++k) q[4 * m + k] = r[k];
         }
-        // scores: quarter wq of every q head of the group against K row j0 + lane
+        if (tt + kStride < t1) load_q(tt + kStride, qraw);
+        float sc[16];  // position 4 i + g of row n
 #pragma unroll
-        for (int g = 0; g < G; ++g) {
-            float a = 0.0f;
+        for (int t = 0; t < 4; ++t) {
+            v4f a[4];
 #pragma unroll
-            for (int i = 0; i < kQP; ++i) {
-                const uint32_t w = qc[g * kQP + i];
-                a = __builtin_fmaf(__uint_as_float(w << 16), kf[2 * i], a);
-                a = __builtin_fmaf(__uint_as_float(w & 0xFFFF0000u), kf[2 * i + 1], a);
-            }
-            red[wq][g][lane] = a;
-        }
-        __syncthreads();  // red complete; the previous token's reads of sc are done
-        if (kPrefetchQ && t + 1 < t1) load_q(t + 1, qn);
-        split_softmax<G>(sc, hmax, hsum, jn, [&](int g, int p) {
-            return ((red[0][g][p] + red[1][g][p]) + (red[2][g][p] + red[3][g][p])) * scale;
-        });
-        __syncthreads();
-        // weighted V sums of the heads o / kVP, element pair dp (all 64
-        // positions without a bound per step in the common full split)
-        for (int o = tid; o < G * kVP; o += kAttnThreads) {
-            const int g = o / kVP;
-            float a0 = 0.0f, a1 = 0.0f;
-            auto step = [&](float e, uint32_t w) {
-                a0 = __builtin_fmaf(e, __uint_as_float(w << 16), a0);
-                a1 = __builtin_fmaf(e, __uint_as_float(w & 0xFFFF0000u), a1);
-            };
-            if (jn == kAttnSplit) {
+            for (int w = 0; w < 4; ++w) a[w] = (v4f){0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-                for (int q = 0; q < kAttnSplit / 4; ++q) {
-                    const float4 e = *reinterpret_cast<const float4*>(&sc[g][4 * q]);
-                    step(e.x, vcol[4 * q]);
-                    step(e.y, vcol[4 * q + 1]);
-                    step(e.z, vcol[4 * q + 2]);
-                    step(e.w, vcol[4 * q + 3]);
+            for (int i = 0; i < kQS; ++i)
+#pragma unroll
+                for (int w = 0; w < 4; ++w) {
+                    const int st = w * kQS + i;
+                    a[w] = __builtin_amdgcn_mfma_f32_16x16x4f32(ks[t][st >> 2][lane][st & 3], q[st],
+                                                                a[w], 0, 0, 0);
                 }
-            } else {
 #pragma unroll
-                for (int jj = 0; jj < kAttnSplit; ++jj)
-                    if (jj < jn) step(sc[g][jj], vcol[jj]);
-            }
-            const int h = kvh * G + g;
-            float* out = pacc + t * hs * HD + (static_cast<long>(h) * S + s) * HD + 2 * dp;
-            *reinterpret_cast<float2*>(out) = make_float2(a0, a1);
-            if (dp == 0) {
-                pm[t * hs + h * S + s] = hmax[g];
-                pl[t * hs + h * S + s] = hsum[g];
-            }
+            for (int v = 0; v < 4; ++v)
+                sc[4 * t + v] = ((a[0][v] + a[1][v]) + (a[2][v] + a[3][v])) * scale;
+        }
+        // softmax of the split (split_softmax's order)
+        const int jn = pos0 + tt + n / G + 1 - j0;  // live positions of row n (any sign, may pass 64)
+        const bool part = pos0 + tt + 1 - j0 < kAttnSplit;  // uniform: some row is masked in part
+        if (part) {
+#pragma unroll
+            for (int i = 0; i < 16; ++i) sc[i] = 4 * i + g < jn ? sc[i] : -INFINITY;
+        }
+        float m = sc[0];
+#pragma unroll
+        for (int i = 1; i < 16; ++i) m = __builtin_fmaxf(m, sc[i]);
+        {
+            float b = m;
+            swap16(m, b);
+            m = __builtin_fmaxf(m, b);
+            b = m;
+            swap32(m, b);
+            m = __builtin_fmaxf(m, b);
+        }
+#pragma unroll
+        for (int i = 0; i < 16; ++i) sc[i] = exp_neg(sc[i] - m);  // 0 where masked (-inf or NaN)
+        float l;
+        {
+            float z[4];
+#pragma unroll
+            for (int t = 0; t < 4; ++t)
+                z[t] = quad_sums(sc[4 * t], sc[4 * t + 1], sc[4 * t + 2], sc[4 * t + 3]);
+            l = quad_sums(z[0], z[1], z[2], z[3]);  // lane group t: sum of tile t
+            float b = l;
+            swap16(l, b);
+            l += b;
+            b = l;
+            swap32(l, b);
+            l += b;
+        }
+        v4f o[kM];
+#pragma unroll
+        for (int e = 0; e < kM; ++e) o[e] = (v4f){0.0f, 0.0f, 0.0f, 0.0f};
+        if (!(part && odd)) {
+#pragma unroll
+            for (int i = 0; i < 16; ++i)
+#pragma unroll
+                for (int e = 0; e < kM; ++e)
+                    o[e] = __builtin_amdgcn_mfma_f32_16x16x4f32(sc[i], vs[i][e >> 2][lane][e & 3],
+                                                                o[e], 0, 0, 0);
+        } else {
+#pragma unroll
+            for (int i = 0; i < 16; ++i)
+#pragma unroll 1
+                for (int k = 0; k < 4; ++k) {
+                    const int jj = 4 * i + k, j = j0 + jj < jlast ? j0 + jj : jlast;
+                    const uint16_t* vr = vc + cache0 + static_cast<long>(j) * HD + kM * n;
+#pragma unroll
+                    for (int v = 0; v < 4; ++v) {
+                        const int row = 4 * g + v;
+                        const float pv = __shfl(sc[i], 16 * k + row, kWave);
+                        if (jj < pos0 + tt + row / G + 1 - j0) {
+#pragma unroll
+                            for (int e = 0; e < kM; ++e)
+                                o[e][v] = __builtin_fmaf(pv, BF16::to_float(vr[e]), o[e][v]);
+                        }
+                    }
+                }
+        }
+        // accumulator v of lane (n, g): row 4 g + v, dims kM n .. kM n + kM - 1.
+        // Unconditional stores (rows that take no part store past the
+        // buffers' extents, which drops them): behind a branch they would
+        // make the next tile's wait for its q wait for them too.
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+            const int row = 4 * g + v, t = tt + row / G, h = kvh * G + row % G;
+            const unsigned at = (static_cast<unsigned>(t) * hs + h * S + s) * HD + kM * n;
+            const unsigned off = t < t1 && pos0 + t >= j0 ? 4 * at : kDropStore;
+#pragma unroll
+            for (int e = 0; e < kM; e += 4)
+                __builtin_amdgcn_raw_buffer_store_b128(
+                    __builtin_bit_cast(u32x4v, (v4f){o[e][v], o[e + 1][v], o[e + 2][v], o[e + 3][v]}),
+                    racc, off + 4 * e, 0, 0);
+        }
+        {
+            const int t = tt + n / G, h = kvh * G + n % G;
+            const unsigned at = static_cast<unsigned>(t) * hs + h * S + s;
+            const unsigned off = g == 0 && t < t1 && pos0 + t >= j0 ? 4 * at : kDropStore;
+            __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(m), rm, off, 0, 0);
+            __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(l), rl, off, 0, 0);
         }
     }
 }
@@ -2790,6 +2905,8 @@ struct PrefillBufs {
     float *pm = nullptr, *pl = nullptr, *pacc = nullptr;
     float* comb = nullptr;      // [chunk][nh * hd] combined attention outputs
     EngineState* st = nullptr;  // [chunk] one decode-state record per token
+    PrefillItem* items = nullptr;  // [max_items] the attention's blocks of a pass
+    size_t max_items = 0;
     int chunk = 0;  // tokens per prefill pass
     // per-token capacities of x, y[0] and y[1..2] (a group's rows of x and y
     // start at its first token * these when a batch's tokens are split into
@@ -2817,6 +2934,9 @@ bool alloc_prefill(PrefillBufs& pf, const spb_model_config& cfg, int S, std::vec
     pf.xrow = static_cast<long>(xmax);
     pf.yrow0 = static_cast<long>(ystack);
     pf.yrow = static_cast<long>(ymax);
+    // at most one item per split and block of one tile per wave
+    const size_t tok = kAttnThreads / kWave * 16 / (nh / cfg.num_key_value_heads);
+    pf.max_items = (C + tok - 1) / tok * S;
     return (pf.x = dev_alloc<int8_t>(C * xmax, own)) && (pf.amax = dev_alloc<float>(C, own)) &&
            (pf.y[0] = dev_alloc<int32_t>(C * ystack, own)) &&
            (pf.y[1] = dev_alloc<int32_t>(C * ymax, own)) &&
@@ -2829,7 +2949,8 @@ bool alloc_prefill(PrefillBufs& pf, const spb_model_config& cfg, int S, std::vec
            (pf.pl = dev_alloc<float>(C * nh * S, own)) &&
            (pf.pacc = dev_alloc<float>(C * nh * S * hd, own)) &&
            (pf.comb = dev_alloc<float>(C * nh * hd, own)) &&
-           (pf.st = dev_alloc<EngineState>(C, own));
+           (pf.st = dev_alloc<EngineState>(C, own)) &&
+           (tokens > 0 || (pf.items = dev_alloc<PrefillItem>(pf.max_items, own)));
 }
 
 SegWeights seg_weights(const spb_sparse_linear* a, const spb_sparse_linear* b,
@@ -2893,20 +3014,46 @@ void launch_attention_hd(int G, dim3 grid, hipStream_t s, const uint16_t* qkv,
     }
 }
 // The prefill form: c tokens at positions pos0 .. pos0 + c - 1 (grid.z).
-constexpr int kPrefillQueries = 16;  // tokens per block of the prefill attention
-
+// The items of a prefill pass over tokens at positions pos0 .. pos0 + c - 1:
+// every (token block, split) pair with a token that reaches the split, so no
+// block is launched for nothing and the XCDs (blocks go to them in turn) get
+// equal shares; a grid of splits x token blocks gave the first XCD 1.14 times
+// (1.44 times in a prompt's first pass) the mean of the live blocks.  A block
+// walks over 1, 2, 4 or 8 tiles per wave: k tiles take about k + 1/2 tile
+// times (its start reads and lays out K and V), and about two blocks at a
+// time share a CU; the k that takes the fewest rounds x tile times wins.
+std::vector<PrefillItem> prefill_items(int G, int nkv, int pos0, int c) {
+    const int tile = kAttnThreads / kWave * (16 / G);
+    std::vector<PrefillItem> best;
+    long best_cost = 0;
+    for (int k = 1; k <= 8; k *= 2) {
+        std::vector<PrefillItem> v;
+        for (int t = 0; t < c; t += k * tile) {
+            const int n = c - t < k * tile ? c - t : k * tile;
+            for (int s = 0; s <= (pos0 + t + n - 1) / kAttnSplit; ++s)
+                v.push_back(PrefillItem{t, n, s, pos0 + t, pos0 + c - 1, 0});
+        }
+        const long slots = 2L * device_cu_count();
+        const long cost = (static_cast<long>(v.size()) * nkv + slots - 1) / slots * (2 * k + 1);
+        if (best.empty() || cost < best_cost) {
+            best.swap(v);
+            best_cost = cost;
+        }
+        if (k * tile >= c) break;
+    }
+    return best;
+}
 template <int HD>
-void launch_attention_prefill_hd(int G, int sp, int nkv, int c, hipStream_t s,
+void launch_attention_prefill_hd(int G, int nitems, int nkv, int c, hipStream_t s,
                                  const uint16_t* qkv, const uint16_t* kc, const uint16_t* vc,
                                  float* pm, float* pl, float* pacc, int max_seq, int S,
-                                 float scale, int pos0, int qkv_stride) {
-    constexpr int Q = kPrefillQueries;
-    const dim3 grid(sp, nkv, (c + Q - 1) / Q), block(kAttnThreads);
+                                 float scale, int qkv_stride, const PrefillItem* items) {
+    const dim3 grid(nitems, nkv), block(kAttnThreads);
     switch (G) {
-    case 1: hipLaunchKernelGGL((attention_prefill_kernel<HD, 1, Q>), grid, block, 0, s, qkv, kc, vc, pm, pl, pacc, max_seq, S, scale, pos0, c, qkv_stride); break;
-    case 2: hipLaunchKernelGGL((attention_prefill_kernel<HD, 2, Q>), grid, block, 0, s, qkv, kc, vc, pm, pl, pacc, max_seq, S, scale, pos0, c, qkv_stride); break;
-    case 4: hipLaunchKernelGGL((attention_prefill_kernel<HD, 4, Q>), grid, block, 0, s, qkv, kc, vc, pm, pl, pacc, max_seq, S, scale, pos0, c, qkv_stride); break;
-    default: hipLaunchKernelGGL((attention_prefill_kernel<HD, 8, Q>), grid, block, 0, s, qkv, kc, vc, pm, pl, pacc, max_seq, S, scale, pos0, c, qkv_stride); break;
+    case 1: hipLaunchKernelGGL((attention_prefill_kernel<HD, 1>), grid, block, 0, s, qkv, kc, vc, pm, pl, pacc, max_seq, S, scale, c, qkv_stride, items); break;
+    case 2: hipLaunchKernelGGL((attention_prefill_kernel<HD, 2>), grid, block, 0, s, qkv, kc, vc, pm, pl, pacc, max_seq, S, scale, c, qkv_stride, items); break;
+    case 4: hipLaunchKernelGGL((attention_prefill_kernel<HD, 4>), grid, block, 0, s, qkv, kc, vc, pm, pl, pacc, max_seq, S, scale, c, qkv_stride, items); break;
+    default: hipLaunchKernelGGL((attention_prefill_kernel<HD, 8>), grid, block, 0, s, qkv, kc, vc, pm, pl, pacc, max_seq, S, scale, c, qkv_stride, items); break;
     }
 }
 
@@ -3136,9 +3283,15 @@ auto vcache = [&](size_t l) { return (*t.vcache)[l] + t.kv_off; };
         hs[t].prompt_len = max_seq;
         hs[t].limit = max_seq;
     }
+    const std::vector<PrefillItem> items = prefill_items(nh / nkv, nkv, pos0, c);
+    const int nitems = static_cast<int>(items.size());
+    if (items.size() > pf.max_items) return hipErrorInvalidValue;
     hipError_t err = hipMemcpyAsync(pf.st, hs.data(), sizeof(EngineState) * c,
                                     hipMemcpyHostToDevice, s);
-    if (err == hipSuccess) err = hipStreamSynchronize(s);  // hs is on this frame
+    if (err == hipSuccess)
+        err = hipMemcpyAsync(pf.items, items.data(), sizeof(PrefillItem) * items.size(),
+                             hipMemcpyHostToDevice, s);
+    if (err == hipSuccess) err = hipStreamSynchronize(s);  // hs and items are on this frame
     if (err != hipSuccess) return err;
     for (size_t l = 0; l < layers.size(); ++l) {
         const spb_transformer_layer& L = layers[l];
@@ -3171,13 +3324,13 @@ auto vcache = [&](size_t l) { return (*t.vcache)[l] + t.kv_off; };
         // splits that some token of the pass reaches
         const int sp = (pos0 + c - 1) / kAttnSplit + 1 < S ? (pos0 + c - 1) / kAttnSplit + 1 : S;
         if (hd == 64)
-            launch_attention_prefill_hd<64>(nh / nkv, sp, nkv, c, s, pf.qkv, kcache(l),
+            launch_attention_prefill_hd<64>(nh / nkv, nitems, nkv, c, s, pf.qkv, kcache(l),
                                             vcache(l), pf.pm, pf.pl, pf.pacc, max_seq, S,
-                                            scale, pos0, qrows + 2 * kvdim);
+                                            scale, qrows + 2 * kvdim, pf.items);
         else
-            launch_attention_prefill_hd<128>(nh / nkv, sp, nkv, c, s, pf.qkv, kcache(l),
+            launch_attention_prefill_hd<128>(nh / nkv, nitems, nkv, c, s, pf.qkv, kcache(l),
                                              vcache(l), pf.pm, pf.pl, pf.pacc, max_seq, S,
-                                             scale, pos0, qrows + 2 * kvdim);
+                                             scale, qrows + 2 * kvdim, pf.items);
         {  // the split combine over (head, token), then the o input per token
             launch_attn_combine(hd, nh, sp, s, pf.pm, pf.pl, pf.pacc, pf.comb, pf.st, S, c);
             CombinedAttn p{pf.comb, qrows};
