@@ -58,3 +58,27 @@ def test_prefill_attention_non_finite_values(gpu, hd, nkv):
         batched, stepwise = _both(model, 256, _prompt(n, cfg.vocab_size, n))
         same = batched.view(torch.int32) == stepwise.view(torch.int32)
         assert (same | (batched.isnan() & stepwise.isnan())).all()
+
+
+@pytest.mark.parametrize("hd,nkv", [(64, 4), (128, 1)])
+def test_packed_prompts_match_single_sequences(gpu, hd, nkv):
+    """Prompts of several sequences share prefill passes: tokens equal those of
+    each sequence alone, with prompts of one token, of one tile and ones that a
+    pass of 2048 tokens cuts in two."""
+    from spbitnet_amd.model import BatchInferenceEngine, InferenceEngine, Model
+    cfg = _small_config(num_key_value_heads=nkv, head_dim=hd, hidden_size=8 * hd,
+                        max_position_embeddings=2048)
+    model = Model.random(cfg, seed=hd + nkv)
+    for lin in ("q_proj", "k_proj"):
+        for l in model.layers:
+            getattr(l, lin).gamma *= 0.05
+    lens = [1, 2, 17, 66, 700, 5, 1, 1500, 130, 900]
+    prompts = [_prompt(n, cfg.vocab_size, i) for i, n in enumerate(lens)]
+    eng = BatchInferenceEngine(model, max_seq=1600, batch=12)
+    got = eng.generate(prompts, 8, stop_at_eos=False)
+    eng.close()
+    one = InferenceEngine(model, max_seq=1600)
+    one.set_prefill_batch(0)
+    for i, p in enumerate(prompts):
+        assert got[i] == one.generate(p, 8, stop_at_eos=False), lens[i]
+    one.close()
