@@ -3152,6 +3152,24 @@ void launch_attn_combine(int hd, int nh, int splits, hipStream_t s, const float*
         launch_attn_combine_hd<128>(nh, splits, s, pm, pl, pacc, comb, st, S, B);
 }
 
+// The o projection's quantised input of B tokens from the partials of the
+// attention's first `splits` splits: the split combine over (head, token),
+// then one block per token; with few splits the token's block folds them
+// itself (the same operations in the same order), a launch and a trip through
+// memory less.
+void launch_attn_input(int hd, int nh, int splits, hipStream_t s, const float* pm,
+                       const float* pl, const float* pacc, float* comb, const EngineState* st,
+                       int S, int B, int8_t* x, float* amax) {
+    const int n = nh * hd;
+    if (splits <= kFusedCombineSplits) {
+        const AttnCombine p{pm, pl, pacc, hd, S, n, hd == 64 ? 6 : 7};
+        launch_prefill_producer(p, n, st, n, B, x, amax, s);
+        return;
+    }
+    launch_attn_combine(hd, nh, splits, s, pm, pl, pacc, comb, st, S, B);
+    launch_prefill_producer(CombinedAttn{comb, n}, n, st, n, B, x, amax, s);
+}
+
 // The first `splits` splits of S (the partials' stride stays S).
 void launch_attention(int hd, int G, int S, int splits, int nkv, hipStream_t s,
                       const uint16_t* qkv, const uint16_t* kc, const uint16_t* vc, float* pm,
@@ -3364,11 +3382,7 @@ hipError_t enqueue_prefill_pass(const PrefillTarget& t, const PrefillBufs& pf,
                                              (*t.kcache)[l], (*t.vcache)[l], pf.pm, pf.pl, pf.pacc,
                                              max_seq, S, scale, qrows + 2 * kvdim, t.kv_stride,
                                              pf.items);
-        {  // the split combine over (head, token), then the o input per token
-            launch_attn_combine(hd, nh, sp, s, pf.pm, pf.pl, pf.pacc, pf.comb, pf.st, S, c);
-            CombinedAttn p{pf.comb, qrows};
-            launch_prefill_producer(p, qrows, pf.st, qrows, c, pf.x, pf.amax, s);
-        }
+        launch_attn_input(hd, nh, sp, s, pf.pm, pf.pl, pf.pacc, pf.comb, pf.st, S, c, pf.x, pf.amax);
         {
             const spb_sparse_linear* o1[1] = {&L.o_proj};
             SegBf16Sink sink{pf.o, L.o_proj.gamma, L.o_proj.gamma, L.o_proj.gamma, H, H,
@@ -4109,12 +4123,8 @@ struct spb_batch_engine {
             }
             launch_attention_batch(hd, nh / nkv, S, splits, nkv, B, s, qkv, kc, vc, pm, pl, pacc,
                                    stb, max_seq, scale, static_cast<int>(qkv_row), kv_seq);
-            {
-                float* const cb = step.comb + static_cast<long>(b0) * qrows;
-                launch_attn_combine(hd, nh, splits, s, pm, pl, pacc, cb, stb, S, B);
-                CombinedAttn p{cb, qrows};
-                launch_prefill_producer(p, qrows, stb, qrows, B, x, amax, s);
-            }
+            launch_attn_input(hd, nh, splits, s, pm, pl, pacc,
+                              step.comb + static_cast<long>(b0) * qrows, stb, S, B, x, amax);
             {
                 const spb_sparse_linear* o1[1] = {&L.o_proj};
                 SegBf16Sink sink{o, L.o_proj.gamma, L.o_proj.gamma, L.o_proj.gamma, H, H,

@@ -1,0 +1,274 @@
+// gemm_wide.hpp -- the 2:4 sparse int8 GEMM for many tokens on the int8
+// structured-sparse matrix cores of gfx950 (v_smfmac_i32_16x16x128_i8):
+//   Y[t][r] = sum_c W[r][c] * X[t][c] (exact int32), X token-major int8.
+// W comes either in spbitnet's packed ternary format (WideTernary) or in the
+// tile order of sparse_i8.hip (WideTiles); the epilogue policy is that of
+// gemm_staged.hpp.
+//
+// Tile: 256 rows x 128 tokens per block of four waves (each 128 rows x 64
+// tokens: 8 strips x 4 tiles of 16 x 16, 128 accumulator registers), two
+// blocks per CU.  K goes in steps of 128 columns through two LDS buffers of 36
+// KB in operand order: a lane's operand is 16 (values), 4 (index word) or
+// 2 x 16 (activations) bytes at its own place, so every LDS access is
+// consecutive over the wave.
+//   * A is decoded once per block into LDS instead of by every wave that uses
+//     it (27 VALU instructions of 4 cycles per strip and step): 16 strips per
+//     step over four SIMDs are ~430 cycles next to the 512 of its 128 SMFMACs.
+//   * A lane's 16-byte load of the bitmaps is one row's four lane groups of
+//     one step; the four lane groups hold four steps, and exchanging them
+//     (transpose) gives every lane its own words of four steps.
+#pragma once
+
+#include "gemm_staged.hpp"
+
+namespace spb {
+namespace {
+
+constexpr int kWideRows = 256, kWideTok = 128, kWideThreads = 256;
+constexpr int kWideStrips = kWideRows / 16, kWideTiles = kWideTok / 16;
+constexpr int kWideWaves = kWideThreads / kWave;
+constexpr int kWideOwn = kWideStrips / kWideWaves;  // strips a wave loads and decodes
+
+struct WideLds {
+    v4i a[2][kWideStrips][kWave];         // 16 compressed values
+    int idx[2][kWideStrips][kWave];       // index words
+    u32x4v b[2][kWideTiles][2][kWave];    // activations: K 16 q + [0, 16), 64 + 16 q + [0, 16)
+};
+
+__device__ __forceinline__ void wide_swap16(uint32_t& a, uint32_t& b) {
+    const auto r = __builtin_amdgcn_permlane16_swap(a, b, false, false);
+    a = r[0];
+    b = r[1];
+}
+__device__ __forceinline__ void wide_swap32(uint32_t& a, uint32_t& b) {
+    const auto r = __builtin_amdgcn_permlane32_swap(a, b, false, false);
+    a = r[0];
+    b = r[1];
+}
+// Register c of lane group g becomes register g of lane group c.
+__device__ __forceinline__ void wide_transpose(uint32_t (&r)[4]) {
+    wide_swap16(r[0], r[1]);
+    wide_swap16(r[2], r[3]);
+    wide_swap32(r[0], r[2]);
+    wide_swap32(r[1], r[3]);
+}
+
+// The packed ternary rows (cols % 128 == 0, 16-byte aligned bitmap rows and
+// 8-byte aligned sign rows; stacked matrices whose boundaries are multiples of
+// 16 rows).  Loads cover four steps.
+struct WideTernary {
+    static constexpr int kAhead = 4;  // steps per load
+    const uint32_t* meta;
+    const uint32_t* values;
+    int rows, ms, vs;
+    GemmSegs segs;
+    struct Raw {
+        u32x4v m[kWideOwn];
+        uint2 v[kWideOwn];
+    };
+    struct Held {
+        uint32_t m[kWideOwn][4], v[kWideOwn][4];
+    };
+    // Steps step0 .. step0 + 3 of strips strip0 .. strip0 + 3: rows past the
+    // matrix and steps past the row's end read zeros or the next row's words
+    // and feed no stored result.
+    __device__ void load(Raw& r, int strip0, int step0, int lane) const {
+        const int st = step0 + (lane >> 4), li = lane & 15;
+        const int om = (li * ms + 4 * st) * 4, ov = (li * vs + 2 * st) * 4;
+#pragma unroll
+        for (int k = 0; k < kWideOwn; ++k) {
+            const int s16 = __builtin_amdgcn_readfirstlane((strip0 + k) * 16);  // in one matrix
+            long om1 = 0, ov1 = 0;
+            if (s16 >= segs.end0) om1 = segs.om1, ov1 = segs.ov1;
+            if (s16 >= segs.end1) om1 = segs.om2, ov1 = segs.ov2;
+            const int nr = max(0, min(rows - s16, 16));
+            const long row = nr ? s16 : 0;
+            const __amdgpu_buffer_rsrc_t rm = __builtin_amdgcn_make_buffer_rsrc(
+                const_cast<uint32_t*>(meta + om1 + row * ms), static_cast<short>(0), nr * ms * 4,
+                kRawBufferFlags);
+            const __amdgpu_buffer_rsrc_t rv = __builtin_amdgcn_make_buffer_rsrc(
+                const_cast<uint32_t*>(values + ov1 + row * vs), static_cast<short>(0), nr * vs * 4,
+                kRawBufferFlags);
+            r.m[k] = __builtin_amdgcn_raw_buffer_load_b128(rm, om, 0, 0);
+            r.v[k] = __builtin_bit_cast(uint2, __builtin_amdgcn_raw_buffer_load_b64(rv, ov, 0, 0));
+        }
+    }
+    __device__ static void hold(const Raw& r, Held& h) {
+#pragma unroll
+        for (int k = 0; k < kWideOwn; ++k) {
+            h.m[k][0] = r.m[k][0], h.m[k][1] = r.m[k][1];
+            h.m[k][2] = r.m[k][2], h.m[k][3] = r.m[k][3];
+            wide_transpose(h.m[k]);
+            // the low 16 bits are the lane's signs
+            h.v[k][0] = r.v[k].x, h.v[k][1] = r.v[k].x >> 16;
+            h.v[k][2] = r.v[k].y, h.v[k][3] = r.v[k].y >> 16;
+            wide_transpose(h.v[k]);
+        }
+    }
+    // strip k's operand of the i-th held step
+    __device__ static void operand(const Held& h, int k, int i, v4i& a, int& idx) {
+        idx = smfmac_index(h.m[k][i]);
+        a = smfmac_values(h.v[k][i]);
+    }
+};
+
+// The tile order of sparse_i8.hip: strip s, step j at byte (s * steps + j) *
+// 1280, values then index words, both by lane.
+struct WideTiles {
+    static constexpr int kAhead = 1;
+    const uint8_t* comp;
+    int strips, steps;
+    struct Raw {
+        v4i a[kWideOwn];
+        int idx[kWideOwn];
+    };
+    using Held = Raw;
+    __device__ void load(Raw& r, int strip0, int step0, int lane) const {
+        const int st = min(step0, steps - 1);
+#pragma unroll
+        for (int k = 0; k < kWideOwn; ++k) {
+            const uint8_t* t =
+                comp + (static_cast<long>(min(strip0 + k, strips - 1)) * steps + st) * 1280;
+            r.a[k] = *reinterpret_cast<const v4i*>(t + 16 * lane);
+            r.idx[k] = *reinterpret_cast<const int*>(t + 1024 + 4 * lane);
+        }
+    }
+    __device__ static void hold(const Raw& r, Held& h) { h = r; }
+    __device__ static void operand(const Held& h, int k, int, v4i& a, int& idx) {
+        a = h.a[k];
+        idx = h.idx[k];
+    }
+};
+
+// xstride: bytes per token of X (a multiple of 16, below 2^23; X 16-byte
+// aligned).  A step may read past a token's bytes where A is zero
+// (WideTiles); past the block's last token the loads return zeros.
+template <class A, class Epi>
+__global__ __launch_bounds__(kWideThreads, 2) void gemm_wide_kernel(A src,
+                                                                    const int8_t* __restrict__ X,
+                                                                    Epi epi, int rows, int nsteps,
+                                                                    int n, int xstride) {
+    extern __shared__ __align__(16) uint8_t wide_smem[];
+    WideLds& sh = *reinterpret_cast<WideLds*>(wide_smem);
+    const int tid = threadIdx.x, lane = tid & (kWave - 1);
+    const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
+    const int q = lane >> 4, li = lane & 15;
+    const int r0 = blockIdx.x * kWideRows, t0 = blockIdx.y * kWideTok;
+    const int ws = wave & 1, wt = wave >> 1;  // the wave's half of the strips and of the tiles
+    // activations: wave w stages tiles 2w and 2w + 1, both 64-byte halves
+    const __amdgpu_buffer_rsrc_t rx = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<int8_t*>(X + static_cast<long>(t0) * xstride), static_cast<short>(0),
+        min(n - t0, kWideTok) * xstride, kRawBufferFlags);
+    const int xo = (32 * wave + li) * xstride + 16 * q;
+    u32x4v xr[2][2];
+    auto load_b = [&](int s) {
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+            for (int h = 0; h < 2; ++h)
+                xr[i][h] = __builtin_amdgcn_raw_buffer_load_b128(
+                    rx, xo + 16 * i * xstride + 128 * s + 64 * h, 0, 0);
+    };
+    auto store_b = [&](int buf) {
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+            for (int h = 0; h < 2; ++h) sh.b[buf][2 * wave + i][h][lane] = xr[i][h];
+    };
+    typename A::Raw raw;
+    typename A::Held held;
+    const int strip0 = r0 / 16 + kWideOwn * wave;
+    auto store_a = [&](int buf, int i) {
+#pragma unroll
+        for (int k = 0; k < kWideOwn; ++k) {
+            v4i a;
+            int idx;
+            A::operand(held, k, i, a, idx);
+            sh.a[buf][kWideOwn * wave + k][lane] = a;
+            sh.idx[buf][kWideOwn * wave + k][lane] = idx;
+        }
+    };
+    v4i acc[8][4];
+#pragma unroll
+    for (int s = 0; s < 8; ++s)
+#pragma unroll
+        for (int t = 0; t < 4; ++t) acc[s][t] = (v4i){0, 0, 0, 0};
+    auto compute = [&](int buf) {
+        v8i b[4];
+#pragma unroll
+        for (int t = 0; t < 4; ++t) {
+            const u32x4v lo = sh.b[buf][4 * wt + t][0][lane], hi = sh.b[buf][4 * wt + t][1][lane];
+            b[t] = (v8i){(int)lo[0], (int)lo[1], (int)lo[2], (int)lo[3],
+                         (int)hi[0], (int)hi[1], (int)hi[2], (int)hi[3]};
+        }
+#pragma unroll
+        for (int s = 0; s < 8; ++s) {
+            const v4i a = sh.a[buf][8 * ws + s][lane];
+            const int idx = sh.idx[buf][8 * ws + s][lane];
+#pragma unroll
+            for (int t = 0; t < 4; ++t)
+                acc[s][t] = __builtin_amdgcn_smfmac_i32_16x16x128_i8(a, b[t], acc[s][t], idx, 0, 0);
+        }
+    };
+    // Step s from buffer i & 1 (i = s % 4), while s + 1 is loaded and laid out
+    // in the other; past the last step that is done for nothing, so that a
+    // step has no branch.
+    auto step = [&](int s, int i) {
+        load_b(s + 1);
+        if (A::kAhead == 4 && i == 2) src.load(raw, strip0, s + 2, lane);
+        if (A::kAhead == 1) {
+            A::hold(raw, held);
+            src.load(raw, strip0, s + 2, lane);
+        }
+        __builtin_amdgcn_sched_barrier(0);  // the loads go out here, not where they are used
+        if (A::kAhead == 4 && i == 3) A::hold(raw, held);
+        store_a((i + 1) & 1, A::kAhead == 4 ? (i + 1) & 3 : 0);
+        compute(i & 1);
+        store_b((i + 1) & 1);
+        __syncthreads();
+    };
+
+    src.load(raw, strip0, 0, lane);
+    load_b(0);
+    A::hold(raw, held);
+    store_a(0, 0);
+    store_b(0);
+    if constexpr (A::kAhead == 1) src.load(raw, strip0, 1, lane);
+    __syncthreads();
+    int s = 0;
+    for (; s + 4 <= nsteps; s += 4) {
+        step(s, 0);
+        step(s + 1, 1);
+        step(s + 2, 2);
+        step(s + 3, 3);
+    }
+    if (s < nsteps) step(s, 0);  // uniform
+    if (s + 1 < nsteps) step(s + 1, 1);
+    if (s + 2 < nsteps) step(s + 2, 2);
+    // lane (li, q) of tile (s, t) holds rows 16 (8 ws + s) + 4q .. + 3 of token 16 (4 wt + t) + li
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+        const int row = r0 + 16 * (8 * ws + e) + 4 * q;
+#pragma unroll
+        for (int t = 0; t < 4; ++t) {
+            const int tok = t0 + 16 * (4 * wt + t) + li;
+            if (tok < n && row < rows) epi.store4(tok, row, acc[e][t], epi.preload(tok, row));
+        }
+    }
+}
+
+template <class A, class Epi>
+int launch_wide(const A& src, const int8_t* X, const Epi& epi, int rows, int nsteps, int n,
+                int xstride, hipStream_t st) {
+    const void* fn = reinterpret_cast<const void*>(&gemm_wide_kernel<A, Epi>);
+    const int lds = static_cast<int>(sizeof(WideLds));
+    if (lds > device_lds_per_cu() || !gemm_allow_lds(fn))
+        return invalid("gemm_wide: %d bytes of LDS unavailable", lds);
+    hipLaunchKernelGGL((gemm_wide_kernel<A, Epi>),
+                       dim3((rows + kWideRows - 1) / kWideRows, (n + kWideTok - 1) / kWideTok),
+                       dim3(kWideThreads), lds, st, src, X, epi, rows, nsteps, n, xstride);
+    return 0;
+}
+
+}  // namespace
+}  // namespace spb
