@@ -5,26 +5,32 @@
 // tile order of sparse_i8.hip (WideTiles); the epilogue policy is that of
 // gemm_staged.hpp.
 //
-// Tile: 256 rows x 128 tokens per block of four waves (each 128 rows x 64
-// tokens: 8 strips x 4 tiles of 16 x 16, 128 accumulator registers), two
-// blocks per CU.  K goes in steps of 128 columns through two LDS buffers of 36
-// KB in operand order: a lane's operand is 16 (values), 4 (index word) or
-// 2 x 16 (activations) bytes at its own place, so every LDS access is
-// consecutive over the wave.
-//   * A is decoded once per block into LDS instead of by every wave that uses
-//     it (27 VALU instructions of 4 cycles per strip and step): 16 strips per
-//     step over four SIMDs are ~430 cycles next to the 512 of its 128 SMFMACs.
+// Tile: 256 rows x 128 tokens per block of eight waves (each 64 rows x 64
+// tokens: 4 strips x 4 tiles of 16 x 16, 64 accumulator registers), two blocks
+// per CU.  K goes in steps of 128 columns through two LDS buffers of 36 KB in
+// operand order: a lane's operand is 16 (values), 4 (index word) or 2 x 16
+// (activations) bytes at its own place, so every LDS access is consecutive
+// over the wave.
+//   * A is decoded once per block into LDS, not by every wave that uses it.
 //   * A lane's 16-byte load of the bitmaps is one row's four lane groups of
 //     one step; the four lane groups hold four steps, and exchanging them
 //     (transpose) gives every lane its own words of four steps.
+//   * Activations go from memory to LDS without passing registers.
+// What bounds it (cycle counts around the parts of a step, one block on a CU):
+// ~600 cycles per wave of decode (54 VALU instructions, 5 cycles each and two
+// waves per SIMD), ~500 of addresses, exchanges and load issue, ~630 of operand
+// reads and 16 SMFMACs (18 cycles each), ~100 of waiting for loads; SMFMACs and
+// VALU instructions of different waves overlap only in part (7.5 ns per SMFMAC,
+// 1.0-1.3 ns more per VALU instruction in its shadow).  Interleaving them by
+// hand, 128 x 64 tiles per wave and 256 tokens per block ran at the same speed.
 #pragma once
 
-#include "gemm_staged.hpp"
+#include "smfmac.hpp"
 
 namespace spb {
 namespace {
 
-constexpr int kWideRows = 256, kWideTok = 128, kWideThreads = 256;
+constexpr int kWideRows = 256, kWideTok = 128, kWideThreads = 512;
 constexpr int kWideStrips = kWideRows / 16, kWideTiles = kWideTok / 16;
 constexpr int kWideWaves = kWideThreads / kWave;
 constexpr int kWideOwn = kWideStrips / kWideWaves;  // strips a wave loads and decodes
@@ -53,6 +59,19 @@ __device__ __forceinline__ void wide_transpose(uint32_t (&r)[4]) {
     wide_swap32(r[1], r[3]);
 }
 
+// 16 bytes per lane from the resource to LDS at base + 16 lane.
+__device__ __forceinline__ void wide_load_lds(const __amdgpu_buffer_rsrc_t r, int offset,
+                                              uint32_t base) {
+    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tbuffer_load_dwordx4 %0, %1, 0 offen lds"
+                 :
+                 : "v"(offset), "s"(r), "s"(__builtin_amdgcn_readfirstlane(base))
+                 : "memory", "m0");
+}
+// Every load, LDS store and LDS read of the wave is done, then of the block.
+__device__ __forceinline__ void wide_barrier() {
+    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+}
+
 // The packed ternary rows (cols % 128 == 0, 16-byte aligned bitmap rows and
 // 8-byte aligned sign rows; stacked matrices whose boundaries are multiples of
 // 16 rows).  Loads cover four steps.
@@ -69,28 +88,20 @@ struct WideTernary {
     struct Held {
         uint32_t m[kWideOwn][4], v[kWideOwn][4];
     };
-    // Steps step0 .. step0 + 3 of strips strip0 .. strip0 + 3: rows past the
-    // matrix and steps past the row's end read zeros or the next row's words
-    // and feed no stored result.
-    __device__ void load(Raw& r, int strip0, int step0, int lane) const {
-        const int st = step0 + (lane >> 4), li = lane & 15;
-        const int om = (li * ms + 4 * st) * 4, ov = (li * vs + 2 * st) * 4;
+    // Steps step0 .. step0 + 3 of strips strip0 .. strip0 + 3.  Rows past the
+    // matrix read its last row and steps past the row its last step; neither
+    // feeds a stored result.
+    __device__ void load(Raw& r, int strip0, int step0, int nsteps, int lane) const {
+        const int st = min(step0 + (lane >> 4), nsteps - 1);
 #pragma unroll
         for (int k = 0; k < kWideOwn; ++k) {
-            const int s16 = __builtin_amdgcn_readfirstlane((strip0 + k) * 16);  // in one matrix
-            long om1 = 0, ov1 = 0;
-            if (s16 >= segs.end0) om1 = segs.om1, ov1 = segs.ov1;
-            if (s16 >= segs.end1) om1 = segs.om2, ov1 = segs.ov2;
-            const int nr = max(0, min(rows - s16, 16));
-            const long row = nr ? s16 : 0;
-            const __amdgpu_buffer_rsrc_t rm = __builtin_amdgcn_make_buffer_rsrc(
-                const_cast<uint32_t*>(meta + om1 + row * ms), static_cast<short>(0), nr * ms * 4,
-                kRawBufferFlags);
-            const __amdgpu_buffer_rsrc_t rv = __builtin_amdgcn_make_buffer_rsrc(
-                const_cast<uint32_t*>(values + ov1 + row * vs), static_cast<short>(0), nr * vs * 4,
-                kRawBufferFlags);
-            r.m[k] = __builtin_amdgcn_raw_buffer_load_b128(rm, om, 0, 0);
-            r.v[k] = __builtin_bit_cast(uint2, __builtin_amdgcn_raw_buffer_load_b64(rv, ov, 0, 0));
+            const int s16 = (strip0 + k) * 16;  // uniform: the strip lies in one matrix
+            long om = 0, ov = 0;
+            if (s16 >= segs.end0) om = segs.om1, ov = segs.ov1;
+            if (s16 >= segs.end1) om = segs.om2, ov = segs.ov2;
+            const int row = min(s16 + (lane & 15), rows - 1);
+            r.m[k] = *reinterpret_cast<const u32x4v*>(meta + om + (static_cast<long>(row) * ms + 4 * st));
+            r.v[k] = *reinterpret_cast<const uint2*>(values + ov + (static_cast<long>(row) * vs + 2 * st));
         }
     }
     __device__ static void hold(const Raw& r, Held& h) {
@@ -123,7 +134,7 @@ struct WideTiles {
         int idx[kWideOwn];
     };
     using Held = Raw;
-    __device__ void load(Raw& r, int strip0, int step0, int lane) const {
+    __device__ void load(Raw& r, int strip0, int step0, int, int lane) const {
         const int st = min(step0, steps - 1);
 #pragma unroll
         for (int k = 0; k < kWideOwn; ++k) {
@@ -144,7 +155,7 @@ struct WideTiles {
 // aligned).  A step may read past a token's bytes where A is zero
 // (WideTiles); past the block's last token the loads return zeros.
 template <class A, class Epi>
-__global__ __launch_bounds__(kWideThreads, 2) void gemm_wide_kernel(A src,
+__global__ __launch_bounds__(kWideThreads, 4) void gemm_wide_kernel(A src,
                                                                     const int8_t* __restrict__ X,
                                                                     Epi epi, int rows, int nsteps,
                                                                     int n, int xstride) {
@@ -154,26 +165,21 @@ __global__ __launch_bounds__(kWideThreads, 2) void gemm_wide_kernel(A src,
     const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
     const int q = lane >> 4, li = lane & 15;
     const int r0 = blockIdx.x * kWideRows, t0 = blockIdx.y * kWideTok;
-    const int ws = wave & 1, wt = wave >> 1;  // the wave's half of the strips and of the tiles
-    // activations: wave w stages tiles 2w and 2w + 1, both 64-byte halves
+    const int ws = wave & 3, wt = wave >> 2;  // the wave's quarter of the strips and half of the tiles
+    // activations: wave w stages tile w, both 64-byte halves
     const __amdgpu_buffer_rsrc_t rx = __builtin_amdgcn_make_buffer_rsrc(
         const_cast<int8_t*>(X + static_cast<long>(t0) * xstride), static_cast<short>(0),
         min(n - t0, kWideTok) * xstride, kRawBufferFlags);
-    const int xo = (32 * wave + li) * xstride + 16 * q;
-    u32x4v xr[2][2];
-    auto load_b = [&](int s) {
+    const int xo = (16 * wave + li) * xstride + 16 * q;
+    // Straight to LDS (lane l's 16 bytes at M0 + 16 l): no registers to hold
+    // the tile over a step, no LDS store instructions.
+    const uint32_t lds_b = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(
+        (__attribute__((address_space(3))) void*)&sh.b[0][wave][0][0]));
+    auto load_b = [&](int s, int buf) {
 #pragma unroll
-        for (int i = 0; i < 2; ++i)
-#pragma unroll
-            for (int h = 0; h < 2; ++h)
-                xr[i][h] = __builtin_amdgcn_raw_buffer_load_b128(
-                    rx, xo + 16 * i * xstride + 128 * s + 64 * h, 0, 0);
-    };
-    auto store_b = [&](int buf) {
-#pragma unroll
-        for (int i = 0; i < 2; ++i)
-#pragma unroll
-            for (int h = 0; h < 2; ++h) sh.b[buf][2 * wave + i][h][lane] = xr[i][h];
+        for (int h = 0; h < 2; ++h)
+            wide_load_lds(rx, xo + 128 * s + 64 * h,
+                          lds_b + buf * sizeof(sh.b[0]) + h * sizeof(sh.b[0][0][0]));
     };
     typename A::Raw raw;
     typename A::Held held;
@@ -188,53 +194,52 @@ __global__ __launch_bounds__(kWideThreads, 2) void gemm_wide_kernel(A src,
             sh.idx[buf][kWideOwn * wave + k][lane] = idx;
         }
     };
-    v4i acc[8][4];
+    v4i acc[4][4];
 #pragma unroll
-    for (int s = 0; s < 8; ++s)
+    for (int s = 0; s < 4; ++s)
 #pragma unroll
         for (int t = 0; t < 4; ++t) acc[s][t] = (v4i){0, 0, 0, 0};
     auto compute = [&](int buf) {
-        v8i b[4];
+        v4i a[4];
+        int idx[4];
+#pragma unroll
+        for (int s = 0; s < 4; ++s) {
+            a[s] = sh.a[buf][4 * ws + s][lane];
+            idx[s] = sh.idx[buf][4 * ws + s][lane];
+        }
 #pragma unroll
         for (int t = 0; t < 4; ++t) {
             const u32x4v lo = sh.b[buf][4 * wt + t][0][lane], hi = sh.b[buf][4 * wt + t][1][lane];
-            b[t] = (v8i){(int)lo[0], (int)lo[1], (int)lo[2], (int)lo[3],
-                         (int)hi[0], (int)hi[1], (int)hi[2], (int)hi[3]};
-        }
+            const v8i b = (v8i){(int)lo[0], (int)lo[1], (int)lo[2], (int)lo[3],
+                                (int)hi[0], (int)hi[1], (int)hi[2], (int)hi[3]};
 #pragma unroll
-        for (int s = 0; s < 8; ++s) {
-            const v4i a = sh.a[buf][8 * ws + s][lane];
-            const int idx = sh.idx[buf][8 * ws + s][lane];
-#pragma unroll
-            for (int t = 0; t < 4; ++t)
-                acc[s][t] = __builtin_amdgcn_smfmac_i32_16x16x128_i8(a, b[t], acc[s][t], idx, 0, 0);
+            for (int s = 0; s < 4; ++s)
+                acc[s][t] = __builtin_amdgcn_smfmac_i32_16x16x128_i8(a[s], b, acc[s][t], idx[s], 0, 0);
         }
     };
     // Step s from buffer i & 1 (i = s % 4), while s + 1 is loaded and laid out
     // in the other; past the last step that is done for nothing, so that a
     // step has no branch.
     auto step = [&](int s, int i) {
-        load_b(s + 1);
-        if (A::kAhead == 4 && i == 2) src.load(raw, strip0, s + 2, lane);
+        load_b(s + 1, (i + 1) & 1);
+        if (A::kAhead == 4 && i == 2) src.load(raw, strip0, s + 2, nsteps, lane);
         if (A::kAhead == 1) {
             A::hold(raw, held);
-            src.load(raw, strip0, s + 2, lane);
+            src.load(raw, strip0, s + 2, nsteps, lane);
         }
         __builtin_amdgcn_sched_barrier(0);  // the loads go out here, not where they are used
         if (A::kAhead == 4 && i == 3) A::hold(raw, held);
         store_a((i + 1) & 1, A::kAhead == 4 ? (i + 1) & 3 : 0);
         compute(i & 1);
-        store_b((i + 1) & 1);
-        __syncthreads();
+        wide_barrier();
     };
 
-    src.load(raw, strip0, 0, lane);
-    load_b(0);
+    src.load(raw, strip0, 0, nsteps, lane);
+    load_b(0, 0);
     A::hold(raw, held);
     store_a(0, 0);
-    store_b(0);
-    if constexpr (A::kAhead == 1) src.load(raw, strip0, 1, lane);
-    __syncthreads();
+    if constexpr (A::kAhead == 1) src.load(raw, strip0, 1, nsteps, lane);
+    wide_barrier();
     int s = 0;
     for (; s + 4 <= nsteps; s += 4) {
         step(s, 0);
@@ -247,8 +252,8 @@ __global__ __launch_bounds__(kWideThreads, 2) void gemm_wide_kernel(A src,
     if (s + 2 < nsteps) step(s + 2, 2);
     // lane (li, q) of tile (s, t) holds rows 16 (8 ws + s) + 4q .. + 3 of token 16 (4 wt + t) + li
 #pragma unroll
-    for (int e = 0; e < 8; ++e) {
-        const int row = r0 + 16 * (8 * ws + e) + 4 * q;
+    for (int e = 0; e < 4; ++e) {
+        const int row = r0 + 16 * (4 * ws + e) + 4 * q;
 #pragma unroll
         for (int t = 0; t < 4; ++t) {
             const int tok = t0 + 16 * (4 * wt + t) + li;
@@ -258,16 +263,36 @@ __global__ __launch_bounds__(kWideThreads, 2) void gemm_wide_kernel(A src,
 }
 
 template <class A, class Epi>
+const void* wide_fn() {
+    return reinterpret_cast<const void*>(&gemm_wide_kernel<A, Epi>);
+}
+
+template <class A, class Epi>
 int launch_wide(const A& src, const int8_t* X, const Epi& epi, int rows, int nsteps, int n,
                 int xstride, hipStream_t st) {
-    const void* fn = reinterpret_cast<const void*>(&gemm_wide_kernel<A, Epi>);
     const int lds = static_cast<int>(sizeof(WideLds));
-    if (lds > device_lds_per_cu() || !gemm_allow_lds(fn))
+    if (lds > device_lds_per_cu() || !gemm_allow_lds(wide_fn<A, Epi>()))
         return invalid("gemm_wide: %d bytes of LDS unavailable", lds);
     hipLaunchKernelGGL((gemm_wide_kernel<A, Epi>),
                        dim3((rows + kWideRows - 1) / kWideRows, (n + kWideTok - 1) / kWideTok),
                        dim3(kWideThreads), lds, st, src, X, epi, rows, nsteps, n, xstride);
     return 0;
+}
+
+long wide_blocks(int rows, int n) {
+    return static_cast<long>((rows + kWideRows - 1) / kWideRows) * ((n + kWideTok - 1) / kWideTok);
+}
+
+// The packed ternary product takes the wide kernel when its grid is 1.5 blocks
+// per CU or more (two fit a CU): below that a block per CU runs at its own
+// latency, ~1 us per 128 columns, and the staged tiles win.  us per launch,
+// staged -> wide: 13824 x 2560, n = 1024 / 2048 / 3000 (432 / 864 / 1296
+// blocks) 53.8 -> 45.7, 104.6 -> 86.6, 147.0 -> 129.6; 6912 x 2560, n = 2048
+// (432) 52.6 -> 46.5; 3840 x 2560, n = 3000 (360) 43.7 -> 43.4, n = 2048 (240)
+// 30.9 -> 31.1; 2560 x 6912, n = 2048 (160) 59.8 -> 65.2.
+bool wide_ternary_ok(int rows, int cols, int n, const GemmSegs& g) {
+    return 2 * wide_blocks(rows, n) >= 3L * device_cu_count() && cols < (1 << 23) &&
+           (g.end0 >= rows || g.end0 % 16 == 0) && (g.end1 >= rows || g.end1 % 16 == 0);
 }
 
 }  // namespace

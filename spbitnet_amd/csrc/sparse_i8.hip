@@ -33,13 +33,11 @@
 // column-major (= [n][m]), as the reference declares them
 // (src/cusparselt_backend.cu:53-78).
 #include "common.hpp"
+#include "gemm_staged.hpp"
 #include "spbitnet_amd.h"
 
 namespace spb {
 namespace {
-
-typedef int v4i __attribute__((ext_vector_type(4)));
-typedef int v8i __attribute__((ext_vector_type(8)));
 
 constexpr int kI8TileBytes = 1280;  // 16 rows x 128 columns: values then index words
 constexpr int kI8ValBytes = 1024;
@@ -164,30 +162,52 @@ __global__ __launch_bounds__(W * kWave) void sparse_i8_gemm_kernel(
     for (int s = 0; s < S; ++s)
 #pragma unroll
         for (int t = 0; t < T; ++t) acc[s][t] = (v4i){0, 0, 0, 0};
-    for (int j = wave; j < steps; j += W) {
-        v4i av[S];
+    // a step's operands, loaded one step ahead of their products: strips past
+    // the matrix read its last one (their rows are not stored), and the loads
+    // past a wave's last step read a step again
+    struct Step {
+        v4i a[S];
         int idx[S];
+        v4i lo[T], hi[T];
+    };
+    auto load = [&](int j, Step& o) {
+        j = j < steps ? j : steps - 1;
 #pragma unroll
         for (int s = 0; s < S; ++s) {
-            av[s] = (v4i){0, 0, 0, 0};
-            idx[s] = 0x44444444;
-            if (s0 + s < strips) {
-                const uint8_t* tp = comp + (static_cast<long>(s0 + s) * steps + j) * kI8TileBytes;
-                av[s] = *reinterpret_cast<const v4i*>(tp + lane * 16);
-                idx[s] = *reinterpret_cast<const int*>(tp + kI8ValBytes + lane * 4);
-            }
+            const int strip = s0 + s < strips ? s0 + s : strips - 1;
+            const uint8_t* tp = comp + (static_cast<long>(strip) * steps + j) * kI8TileBytes;
+            o.a[s] = *reinterpret_cast<const v4i*>(tp + lane * 16);
+            o.idx[s] = *reinterpret_cast<const int*>(tp + kI8ValBytes + lane * 4);
         }
 #pragma unroll
         for (int t = 0; t < T; ++t) {
             const int off = (t0 + 16 * t + li) * k + 128 * j + 16 * q;
-            const v4i lo = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(rb, off, 0, 0));
-            const v4i hi =
+            o.lo[t] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(rb, off, 0, 0));
+            o.hi[t] =
                 __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(rb, off + 64, 0, 0));
-            const v8i b = (v8i){lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+        }
+    };
+    auto multiply = [&](const Step& o) {
+#pragma unroll
+        for (int t = 0; t < T; ++t) {
+            const v8i b = (v8i){o.lo[t][0], o.lo[t][1], o.lo[t][2], o.lo[t][3],
+                                o.hi[t][0], o.hi[t][1], o.hi[t][2], o.hi[t][3]};
 #pragma unroll
             for (int s = 0; s < S; ++s)
-                acc[s][t] = __builtin_amdgcn_smfmac_i32_16x16x128_i8(av[s], b, acc[s][t], idx[s], 0, 0);
+                acc[s][t] =
+                    __builtin_amdgcn_smfmac_i32_16x16x128_i8(o.a[s], b, acc[s][t], o.idx[s], 0, 0);
         }
+    };
+    Step x, y;
+    load(wave, x);
+    for (int j = wave; j < steps; j += 2 * W) {
+        load(j + W, y);
+        __builtin_amdgcn_sched_barrier(0);
+        multiply(x);
+        if (j + W >= steps) break;  // uniform
+        load(j + 2 * W, x);
+        __builtin_amdgcn_sched_barrier(0);
+        multiply(y);
     }
     if (W > 1) {
 #pragma unroll
@@ -262,6 +282,38 @@ void launch_i8_gemm(const uint8_t* comp, const int8_t* B, int32_t* D, int m, int
     const int quads = (m % 4 == 0 && i8_aligned(D, 16)) ? 1 : 0;
     hipLaunchKernelGGL((sparse_i8_gemm_kernel<S, T, W>), grid, dim3(W * kWave), 0, st, comp, B, D,
                        m, k, n, steps, strips, quads);
+}
+
+// The tile for n tokens.  us per launch, the 32 x 64 tile without the loads a
+// step ahead that every size above 16 took before -> now:
+//   * a grid of at least 5/8 wide blocks (256 x 128) per CU: the wide kernel.
+//     13824 x 2560, n = 512 / 1024 / 2048 72.8 -> 31.6, 135 -> 44.2, 263 -> 87.5;
+//     6912 x 2560, n = 1024 / 2048 70.2 -> 32.5, 132 -> 45.5; 2560 x 6912,
+//     n = 2048 (160 blocks) 131 -> 67;
+//   * long rows (over 4096 columns) with at least half a 128 x 32 block per
+//     CU: each activation feeds eight strips; 2560 x 6912, n = 256 / 512 / 1024
+//     27.8 -> 14.9, 41.3 -> 25.6, 78.7 -> 37.4 (54.4 with 96 x 32);
+//   * enough 96 x 32 blocks (two per CU): 6912 x 2560, n = 256 / 512 22.3 ->
+//     14.1, 36.7 -> 22.5; 13824 x 2560, n = 128 / 256 23.4 -> 14.0, 38.3 -> 21.7;
+//   * else 64 x 32: 6912 x 2560, n = 128 12.1 -> 9.5; 2560 x 6912, n = 128
+//     15.2 -> 10.7; 2560 x 2560, n = 256 12.0 -> 8.7.
+int launch_i8_for(const uint8_t* comp, const int8_t* B, int32_t* D, int m, int k, int n,
+                  hipStream_t st) {
+    const long cus = device_cu_count(), passes = (n + 31) / 32;
+    if (8 * wide_blocks(m, n) >= 5 * cus) {
+        const WideTiles src{comp, static_cast<int>(i8_strips(m)), static_cast<int>(i8_steps(k))};
+        const Int32Out out{D, m, m % 4 == 0 && i8_aligned(D, 16)};
+        return launch_wide(src, B, out, m, static_cast<int>(i8_steps(k)), n, k, st);
+    }
+    if (n <= 16)
+        launch_i8_gemm<2, 1, 4>(comp, B, D, m, k, n, st);
+    else if (k > 4096 && 2 * ((m + 127) / 128) * passes >= cus)
+        launch_i8_gemm<8, 2, 4>(comp, B, D, m, k, n, st);
+    else if ((m + 95) / 96 * passes >= 2 * cus)
+        launch_i8_gemm<6, 2, 4>(comp, B, D, m, k, n, st);
+    else
+        launch_i8_gemm<4, 2, 4>(comp, B, D, m, k, n, st);
+    return 0;
 }
 
 const char* i8_shape_error(int m, int k) {
@@ -357,12 +409,7 @@ extern "C" int spb_sparse_i8_gemm(const void* compressed, const int8_t* B, int32
     hipStream_t st = as_stream(stream);
     const auto* comp = static_cast<const uint8_t*>(compressed);
     if (spb_sparse_i8_gemm_kernel_id(compressed, B, m, k, n)) {
-        if (n <= 16)
-            launch_i8_gemm<2, 1, 4>(comp, B, D, m, k, n, st);
-        else if (n <= 64)
-            launch_i8_gemm<2, 4, 4>(comp, B, D, m, k, n, st);
-        else
-            launch_i8_gemm<2, 4, 4>(comp, B, D, m, k, n, st);
+        if (const int rc = launch_i8_for(comp, B, D, m, k, n, st)) return rc;
     } else {
         if (n > 65535) return invalid("%s: n = %d exceeds 65535 on the general kernel", fn, n);
         hipLaunchKernelGGL(sparse_i8_gemm_general_kernel,
