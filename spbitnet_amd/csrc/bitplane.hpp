@@ -181,19 +181,16 @@ __device__ __forceinline__ uint32_t q8_biased(float v, float scale) {
         uint32_t, __builtin_amdgcn_fmed3f(v * scale + kBias, kBias - 128.0f, kBias + 127.0f));
 }
 
-// Unit u (columns 8u .. 8u+7) of the activations, 8 floats in registers,
-// quantised and stored into the plane-major LDS planes.  The 4 units of a
+// Unit u (columns 8u .. 8u+7) of the activations, 8 quantised values (their
+// low bytes), stored into the plane-major LDS planes.  The 4 units of a
 // plane word sit in the 4 lanes of a quad (u % 4 == lane % 4 for
 // u = tid + k * kBlock); after the 8x8 bit transpose each lane holds one byte
 // of every plane, and a byte transpose across the quad (two DPP exchanges,
 // lane ^ 1 then lane ^ 2) gives lane q the whole words of planes q and q + 4:
 // two dword stores instead of eight byte stores.  All 4 lanes of a quad run
 // this together.
-__device__ __forceinline__ void store_unit_planes(uint32_t* planes, int nw, int u,
-                                                  const float (&v)[8], float scale) {
-    uint32_t t[8];
-#pragma unroll
-    for (int e = 0; e < 8; ++e) t[e] = q8_biased(v[e], scale);
+__device__ __forceinline__ void store_unit_bytes(uint32_t* planes, int nw, int u,
+                                                 const uint32_t (&t)[8]) {
     // byte e of (lo, hi) = column 8u + e
     uint32_t lo = __builtin_amdgcn_perm(t[1], t[0], 0x0C0C0400u) | __builtin_amdgcn_perm(t[3], t[2], 0x04000C0Cu);
     uint32_t hi = __builtin_amdgcn_perm(t[5], t[4], 0x0C0C0400u) | __builtin_amdgcn_perm(t[7], t[6], 0x04000C0Cu);
@@ -212,6 +209,15 @@ __device__ __forceinline__ void store_unit_planes(uint32_t* planes, int nw, int 
     const int w = u >> 2;
     planes[q * nw + w] = quad_t(lo);
     planes[(q + 4) * nw + w] = quad_t(hi);
+}
+
+// Unit u from 8 floats in registers, quantised.
+__device__ __forceinline__ void store_unit_planes(uint32_t* planes, int nw, int u,
+                                                  const float (&v)[8], float scale) {
+    uint32_t t[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) t[e] = q8_biased(v[e], scale);
+    store_unit_bytes(planes, nw, u, t);
 }
 
 // ---- activation sources ----------------------------------------------------------
@@ -344,6 +350,63 @@ struct GlobalPlanes {
     }
 };
 
+// Planes of 16-bit activations that the block itself quantises with their own
+// absmax (the whole BitLinear in one launch): at most KU 16-byte units per
+// thread, loaded ahead of the weights and kept in registers through the
+// absmax.  The rule and the absmax are QuantSrc's and block_absmax's.
+template <class T, int KU>
+struct AbsmaxPlanes {
+    const uint16_t* x;
+    int units;  // cols / 8 <= KU * kBlock
+    float amax;
+    struct Regs {
+        uint4 r[KU];
+    };
+    static size_t extra_lds(int) { return kBlock / kWave * sizeof(float); }
+    __device__ bool skip() const { return false; }
+    __device__ void offset(long) {}
+    __device__ void prepare() {}
+    __device__ float absmax() const { return amax; }
+    __device__ void issue(int tid, Regs& g) const {
+#pragma unroll
+        for (int k = 0; k < KU; ++k) {  // a thread past the vector reads its last unit again
+            const int u = tid + k * kBlock;
+            g.r[k] = reinterpret_cast<const uint4*>(x)[u < units ? u : units - 1];
+        }
+    }
+    __device__ void build(uint32_t* planes, int cols, int tid, float* slot, const Regs& g) {
+        float f[KU][8], m = 0.0f;
+#pragma unroll
+        for (int k = 0; k < KU; ++k) {
+            const uint32_t w[4] = {g.r[k].x, g.r[k].y, g.r[k].z, g.r[k].w};
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                f[k][e] = T::to_float(static_cast<uint16_t>((e & 1) ? w[e >> 1] >> 16 : w[e >> 1]));
+                m = __builtin_fmaxf(m, __builtin_fabsf(f[k][e]));
+            }
+        }
+        m = wave_max(m);
+        if ((tid & (kWave - 1)) == 0) slot[tid / kWave] = m;
+        __syncthreads();
+        m = slot[0];
+#pragma unroll
+        for (int w = 1; w < kBlock / kWave; ++w) m = __builtin_fmaxf(m, slot[w]);
+        amax = m;
+        const float scale = quant_scale(m);
+#pragma unroll
+        for (int k = 0; k < KU; ++k) {
+            const int u = tid + k * kBlock;
+            if (u < units) {  // whole quads: units is a multiple of 16
+                uint32_t q[8];
+#pragma unroll
+                for (int e = 0; e < 8; ++e)
+                    q[e] = static_cast<uint32_t>(quant_round_clamp(f[k][e] * scale));
+                store_unit_bytes(planes, cols >> 5, u, q);
+            }
+        }
+    }
+};
+
 // ---- output sinks ------------------------------------------------------------------
 
 struct Int32Sink {
@@ -368,6 +431,22 @@ struct DequantSink {
     __device__ void prefetch(long, int, int) {}
     template <class A>
     __device__ void bind(const A&) {}
+    __device__ void store(long r, int acc) const {
+        out[r] = T::from_float(static_cast<float>(acc) * dq);
+    }
+};
+
+// The same with the absmax that the block's activations came with.
+template <class T>
+struct DequantOwnSink {
+    uint16_t* out;
+    float gamma;
+    float dq;
+    __device__ void offset(long) {}
+    __device__ void prepare() {}
+    __device__ void prefetch(long, int, int) {}
+    template <class A>
+    __device__ void bind(const A& a) { dq = dequant_scale(gamma, a.absmax()); }
     __device__ void store(long r, int acc) const {
         out[r] = T::from_float(static_cast<float>(acc) * dq);
     }
