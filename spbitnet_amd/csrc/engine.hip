@@ -59,6 +59,14 @@ constexpr int kGemmSplitCounters = 1024;  // split-K tile counters of a batch en
 // 4,509-4,512 with one, 4,354-4,384 with two).  Larger batches keep one
 // branch, so the GEMMs' split over K (33-64 tokens) sees the whole batch.
 int batch_groups(int batch) { return batch >= 24 && batch <= 32 ? 2 : 1; }
+// ... in the step graphs whose attention reaches more than this many splits
+// (768 positions).  Below, the second branch's launches and its second read of
+// the weights cost more than their overlap with the attention gives.  2B
+// shape, us per step, two groups -> one: 32 sequences at positions 100 / 300 /
+// 500 / 750 1710-1854 -> 1663-1673, 1808 -> 1825, 1959 -> 1941, 2010 -> 2031;
+// at 1000 / 2048 2065 -> 2144, 2544 -> 2657; 24 sequences 1842-1942 -> 1603-
+// 1617, 1743 -> 1739, 1843 -> 1814, 1901 -> 1898, 1922 -> 1979, 2287 -> 2394.
+constexpr int kGroupSplits = 12;
 constexpr long kPrefillPartialBytes = (1L << 31) - 1;  // split partials of one pass (at most)
 constexpr int kPrefillMinDefault = 16;   // prompt tokens before the last that switch to it
 constexpr int kAttnMaxGroup = 8;  // q heads per kv head
@@ -4026,9 +4034,9 @@ struct spb_batch_engine {
     std::vector<float2> rope_host;
     hipStream_t stream = nullptr;
     hipStream_t cap_stream = nullptr;
-    // Sequence groups (batch_groups): the layers of each group of sequences
-    // run as a parallel branch of the step graph (each with its own split-K
-    // workspace), joined before the LM head.  aux: the capture streams of
+    // Sequence groups (batch_groups): past kGroupSplits splits the layers of
+    // each group of sequences run as a parallel branch of the step graph (each
+    // with its own split-K workspace), joined before the LM head.  aux: the capture streams of
     // groups 1 .. groups - 1; ev[0] forks, ev[g] joins group g.
     int groups = 1;
     std::vector<hipStream_t> aux;
@@ -4165,7 +4173,7 @@ struct spb_batch_engine {
     // matrix-core logits over every sequence, then the exact candidates and
     // the argmax per sequence).
     hipError_t enqueue_step(hipStream_t s, int splits) const {
-        if (groups == 1) {
+        if (groups == 1 || splits <= kGroupSplits) {
             const hipError_t err = enqueue_layers(s, 0, batch, splits, &gsplit[0]);
             if (err != hipSuccess) return err;
             return enqueue_head(s);
