@@ -1427,6 +1427,79 @@ __global__ __launch_bounds__(kWave) void attn_combine_kernel(const float* __rest
         out[h * HD + t] = bf16r(a[0] / l);
 }
 
+// The same fold for the many tokens of a prefill pass (token blockIdx.y), where
+// the partials' bytes count and not one head's chain of loads: a wave takes 256
+// / HD heads, 16 bytes per lane and split, eight splits in flight while eight
+// are added.  Operations and order are attn_combine_kernel's.
+// Bound by reading the partials: 4.9 TB/s (3.8 with one wave per head, which
+// loads every split the pass reaches for every token, 8 bytes per lane).
+template <int HD>
+__global__ __launch_bounds__(kWave) void attn_combine_tokens_kernel(
+    const float* __restrict__ pm, const float* __restrict__ pl, const float* __restrict__ pacc,
+    float* __restrict__ out, const EngineState* __restrict__ st, int nh, int S) {
+    constexpr int LH = HD / 4, HW = kWave / LH, NB = 8;  // lanes of a head, heads of the wave
+    extern __shared__ float wl[];                        // [HW][2][S]: w_s, l_s
+    const int hl = threadIdx.x / LH, t = threadIdx.x % LH;
+    const long b = blockIdx.y;
+    const int h = blockIdx.x * HW + hl;
+    const int pos = state_pos(st + b);
+    int ns = (pos >> 6) + 1;
+    ns = ns < S ? ns : S;
+    const long hs = (b * nh + (h < nh ? h : nh - 1)) * S;
+    const float* mh = pm + hs;
+    const float* lh = pl + hs;
+    const float4* ph = reinterpret_cast<const float4*>(pacc + hs * HD) + t;
+    float* w = wl + hl * 2 * S;
+    auto load = [&](int s0, float4 (&v)[NB]) {
+#pragma unroll
+        for (int k = 0; k < NB; ++k)
+            v[k] = ph[static_cast<long>(s0 + k < ns ? s0 + k : ns - 1) * LH];
+    };
+    float4 va[NB], vb[NB];
+    load(0, va);
+    const float m0 = t < ns ? mh[t] : -INFINITY;
+    const float l0 = t < ns ? lh[t] : 0.0f;
+    float M = m0;
+    for (int s = t + LH; s < ns; s += LH) M = __builtin_fmaxf(M, mh[s]);
+    M = __builtin_fmaxf(M, dpp_f<0xB1>(M));
+    M = __builtin_fmaxf(M, dpp_f<0x4E>(M));
+    M = __builtin_fmaxf(M, dpp_f<0x141>(M));
+    M = __builtin_fmaxf(M, dpp_f<0x140>(M));
+    if constexpr (LH == 32) M = __builtin_fmaxf(M, __shfl_xor(M, 16));
+    if (t < ns) {
+        w[t] = exp_neg(m0 - M);
+        w[S + t] = l0;
+    }
+    for (int s = t + LH; s < ns; s += LH) {
+        w[s] = exp_neg(mh[s] - M);
+        w[S + s] = lh[s];
+    }
+    __syncthreads();  // one wave: orders its LDS writes and reads
+    float l = 0.0f, a[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+    auto add = [&](int s0, const float4 (&v)[NB]) {
+#pragma unroll
+        for (int k = 0; k < NB; ++k) {
+            if (s0 + k < ns) {
+                const float e = w[s0 + k];
+                l = __builtin_fmaf(e, w[S + s0 + k], l);
+                a[0] = __builtin_fmaf(e, v[k].x, a[0]);
+                a[1] = __builtin_fmaf(e, v[k].y, a[1]);
+                a[2] = __builtin_fmaf(e, v[k].z, a[2]);
+                a[3] = __builtin_fmaf(e, v[k].w, a[3]);
+            }
+        }
+    };
+    for (int s0 = 0; s0 < ns; s0 += 2 * NB) {
+        if (s0 + NB < ns) load(s0 + NB, vb);
+        add(s0, va);
+        if (s0 + 2 * NB < ns) load(s0 + 2 * NB, va);
+        if (s0 + NB < ns) add(s0 + NB, vb);
+    }
+    if (h < nh)
+        reinterpret_cast<float4*>(out + (b * nh + h) * HD)[t] =
+            make_float4(bf16r(a[0] / l), bf16r(a[1] / l), bf16r(a[2] / l), bf16r(a[3] / l));
+}
+
 template <int HD, int G, int HB = G>
 __global__ __launch_bounds__(kAttnThreads) void attention_kernel(
     const uint16_t* __restrict__ qkv, const uint16_t* __restrict__ kc,
@@ -3149,11 +3222,29 @@ void launch_attn_combine_hd(int nh, int splits, hipStream_t s, const float* pm, 
     }
 #undef SPB_COMBINE_NB
 }
+// From this many tokens on the form for many tokens.  2047 prefill tokens of the
+// 2B shape (32 splits, 335 MB live): 88 -> 68 us per layer, the prefill 21.96 ->
+// 21.38 ms.  Decode steps of 6 layers, us, one wave per head -> this form:
+// 8 sequences at position 2000 475 -> 483, 32 658 -> 669, 64 1077 -> 1080,
+// 128 1887 -> 1881; 256 at 700 2287 -> 2282: the line lies where they meet.
+constexpr int kCombineTokens = 128;
 // B sequences: grid (nh, B), sequence b's state st + b, partials after
 // those of b - 1, output comb + b * nh * hd.
 void launch_attn_combine(int hd, int nh, int splits, hipStream_t s, const float* pm,
                          const float* pl, const float* pacc, float* comb, const EngineState* st,
                          int S, int B = 1) {
+    const int hw = 4 * kWave / hd;  // heads of a wave
+    const size_t lds = 2 * static_cast<size_t>(hw) * S * sizeof(float);
+    if (B >= kCombineTokens && lds <= 65536) {
+        const dim3 grid((nh + hw - 1) / hw, B);
+        if (hd == 64)
+            hipLaunchKernelGGL((attn_combine_tokens_kernel<64>), grid, dim3(kWave), lds, s, pm, pl,
+                               pacc, comb, st, nh, S);
+        else
+            hipLaunchKernelGGL((attn_combine_tokens_kernel<128>), grid, dim3(kWave), lds, s, pm,
+                               pl, pacc, comb, st, nh, S);
+        return;
+    }
     if (hd == 64)
         launch_attn_combine_hd<64>(nh, splits, s, pm, pl, pacc, comb, st, S, B);
     else
