@@ -42,6 +42,13 @@ int launch_status(const char* what) {
     return 0;
 }
 
+int failed(const char* what, hipError_t e) {
+    const hipError_t pending = hipGetLastError();
+    if (e == hipSuccess) e = pending != hipSuccess ? pending : hipErrorUnknown;
+    if (!g_err[0]) set_error("%s: failed: %s", what, hipGetErrorString(e));
+    return static_cast<int>(e);
+}
+
 int device_cu_count() {
     int dev = 0;
     if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= kMaxDevices) return 256;

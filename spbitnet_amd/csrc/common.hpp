@@ -24,6 +24,11 @@ int invalid(const char* fmt, ...);
 // Checks the launch status and records it.
 int launch_status(const char* what);
 
+// The status of an entry point whose step failed with e: never 0, also where
+// a check on the way has already taken HIP's pending error.  Keeps the message
+// that the step recorded.
+int failed(const char* what, hipError_t e);
+
 inline hipStream_t as_stream(void* s) { return reinterpret_cast<hipStream_t>(s); }
 
 // Number of compute units of the current device (cached per device).

@@ -3322,7 +3322,9 @@ struct PrefillTarget {
 // and ld[i]: where projection i's rows are and their row stride.
 hipError_t gemm_group(const spb_sparse_linear* const* w, int nw, const int8_t* X,
                       int32_t* const* y, int n, hipStream_t s, const int32_t** out, int* ld) {
-    if (gemm_stacked(w, nw, X, y[0], n, s) == 0) {
+    const int rc = gemm_stacked(w, nw, X, y[0], n, s);
+    if (rc == 2) return hipErrorLaunchFailure;
+    if (rc == 0) {
         int rows = 0;
         for (int i = 0; i < nw; ++i) rows += w[i]->rows;
         int off = 0;
@@ -3779,7 +3781,7 @@ extern "C" int spb_engine_create(const spb_model_config* cfg, const spb_transfor
     *out = nullptr;
     if (int rc = check_model(fn, cfg, layers, embed_tokens, lm_head, max_seq)) return rc;
     if (gemm_prepare() != 0 || gemm_sink_prepare() != 0)  // before any graph capture
-        return launch_status(fn);
+        return failed(fn, hipSuccess);
     const int H = cfg->hidden_size, nh = cfg->num_attention_heads, nkv = cfg->num_key_value_heads;
     const int hd = cfg->head_dim, I = cfg->intermediate_size, V = cfg->vocab_size;
     const int kvdim = nkv * hd;
@@ -3856,12 +3858,12 @@ extern "C" int spb_engine_create(const spb_model_config* cfg, const spb_transfor
             err = hipStreamBeginCapture(e->cap_stream, hipStreamCaptureModeThreadLocal);
             if (err == hipSuccess) {
                 e->enqueue_step(e->cap_stream, splits);
+                const hipError_t le = hipGetLastError();
                 err = hipStreamEndCapture(e->cap_stream, &g);
+                if (err == hipSuccess) e->graphs.push_back(g);
+                if (err == hipSuccess && le != hipSuccess) err = le;
             }
-            if (err == hipSuccess) {
-                e->graphs.push_back(g);
-                err = hipGraphInstantiate(&x, g, nullptr, nullptr, 0);
-            }
+            if (err == hipSuccess) err = hipGraphInstantiate(&x, g, nullptr, nullptr, 0);
             if (err == hipSuccess) e->execs.push_back(x);
         }
     }
@@ -3969,7 +3971,8 @@ extern "C" int spb_engine_generate(spb_engine* e, const int* prompt, int n_promp
     if (e->prefill_min > 0 && pre >= e->prefill_min) {
         for (int p0 = 0; p0 < pre; p0 += e->pf.chunk) {
             const int c = pre - p0 < e->pf.chunk ? pre - p0 : e->pf.chunk;
-            if (e->enqueue_prefill(p0, c, e->stream) != hipSuccess) return launch_status(fn);
+            const hipError_t err = e->enqueue_prefill(p0, c, e->stream);
+            if (err != hipSuccess) return failed(fn, err);
         }
         if (int rc = set_state(e, pre, n_prompt, stop_at_eos ? 1 : 0)) return rc;
         start = pre;
@@ -4391,19 +4394,21 @@ extern "C" int spb_batch_engine_create(const spb_model_config* cfg,
     }
     if (gemm_prepare() != 0 || gemm_sink_prepare() != 0) {
         delete e;
-        return launch_status(fn);
+        return failed(fn, hipSuccess);
     }
     // the LM-head rows' norms for the error bounds (the table is the model's,
     // unchanged while the engine lives)
     hipLaunchKernelGGL(lm_row_norm_kernel, dim3((V + 3) / 4), dim3(256), 0, nullptr, e->lm_head,
                        e->wnorm, V, H);
-    if (hipGetLastError() != hipSuccess || hipDeviceSynchronize() != hipSuccess) {
+    hipError_t err = hipGetLastError();
+    if (err == hipSuccess) err = hipDeviceSynchronize();
+    if (err != hipSuccess) {
         delete e;
-        return launch_status(fn);
+        return failed(fn, err);
     }
     e->rope_host = rope_table(*cfg, max_seq);
-    hipError_t err = hipMemcpy(e->rope, e->rope_host.data(), e->rope_host.size() * sizeof(float2),
-                               hipMemcpyHostToDevice);
+    err = hipMemcpy(e->rope, e->rope_host.data(), e->rope_host.size() * sizeof(float2),
+                    hipMemcpyHostToDevice);
     for (size_t l = 0; l < e->kcache.size() && err == hipSuccess; ++l) {
         err = hipMemset(e->kcache[l], 0, kv * 2);
         if (err == hipSuccess) err = hipMemset(e->vcache[l], 0, kv * 2);
@@ -4537,15 +4542,16 @@ extern "C" int spb_batch_engine_generate(spb_batch_engine* e, const int* prompts
                 p0 += n;
                 c += n;
                 if (c == e->pf.chunk) {
-                    if (enqueue_prefill_pass(t, e->pf, segs, s) != hipSuccess)
-                        return launch_status(fn);
+                    const hipError_t err = enqueue_prefill_pass(t, e->pf, segs, s);
+                    if (err != hipSuccess) return failed(fn, err);
                     segs.clear();
                     c = 0;
                 }
             }
         }
-        if (c > 0 && enqueue_prefill_pass(t, e->pf, segs, s) != hipSuccess)
-            return launch_status(fn);
+        const hipError_t err =
+            c > 0 ? enqueue_prefill_pass(t, e->pf, segs, s) : hipSuccess;
+        if (err != hipSuccess) return failed(fn, err);
     }
     // decode states: sequence b continues at its last prompt token; unused
     // slots are done
