@@ -399,7 +399,12 @@ typedef struct spb_engine spb_engine;
 
 /* InferenceEngine(const Model&) (inference.h:27): borrows the weights (they
  * must outlive the engine), allocates the KV cache for max_seq positions and
- * scratch, and captures the token-step graph.  embed_tokens / lm_head: bf16
+ * scratch, and captures the token-step graph.  The scratch is mostly that of
+ * the prompts' passes: for the smallest of 2048 tokens, the tokens that
+ * prompts can have and as many as keep the attention's split partials,
+ * 4 * num_attention_heads * ceil(max_seq / 64) * (head_dim + 2) bytes a token,
+ * below 2 GB; half as many, and again, where the device has no room for it.
+ * embed_tokens / lm_head: bf16
  * [vocab][hidden]; lm_head NULL = tied to the embedding. */
 int spb_engine_create(const spb_model_config* config, const spb_transformer_layer* layers,
                       const uint16_t* embed_tokens, const uint16_t* lm_head,

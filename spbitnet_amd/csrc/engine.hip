@@ -2986,7 +2986,10 @@ bool aligned_to(const void* p, uintptr_t a) { return (reinterpret_cast<uintptr_t
 template <class T>
 T* dev_alloc(size_t n, std::vector<void*>& owned) {
     void* p = nullptr;
-    if (hipMalloc(&p, n * sizeof(T) < 16 ? 16 : n * sizeof(T)) != hipSuccess) return nullptr;
+    if (hipMalloc(&p, n * sizeof(T) < 16 ? 16 : n * sizeof(T)) != hipSuccess) {
+        (void)hipGetLastError();  // the caller reports it, not a later launch's check
+        return nullptr;
+    }
     owned.push_back(p);
     return static_cast<T*>(p);
 }
@@ -3009,19 +3012,13 @@ struct PrefillBufs {
     long xrow = 0, yrow0 = 0, yrow = 0;
 };
 
-// The batched prefill's buffers, for nseq sequences: up to kPrefillChunk tokens per pass, fewer
-// when the split partials of a pass would exceed kPrefillPartialBytes; or,
-// with tokens > 0, exactly that many (the batched decode step's buffers).
-bool alloc_prefill(PrefillBufs& pf, const spb_model_config& cfg, int S, std::vector<void*>& own,
-                   int nseq, int tokens = 0) {
+// Buffers of C tokens per pass for nseq sequences (items: those of a prompt's
+// passes too); false when the device has no room, with what was allocated in own.
+bool alloc_pass(PrefillBufs& pf, const spb_model_config& cfg, int S, std::vector<void*>& own,
+                size_t C, size_t nseq, bool items) {
     const int H = cfg.hidden_size, nh = cfg.num_attention_heads, hd = cfg.head_dim;
     const int I = cfg.intermediate_size, kvdim = cfg.num_key_value_heads * hd;
-    const long part = static_cast<long>(nh) * S * (hd + 2) * 4;  // bytes per token
-    long c = kPrefillPartialBytes / part;
-    c = c < kPrefillChunk ? c : kPrefillChunk;
-    if (tokens > 0) c = tokens;
-    pf.chunk = static_cast<int>(c > 0 ? c : 1);
-    const size_t C = static_cast<size_t>(pf.chunk);
+    pf.chunk = static_cast<int>(C);
     const size_t xmax = static_cast<size_t>(std::max(std::max(H, I), nh * hd));
     // y[0] also holds the stacked q|k|v and gate|up products
     const size_t ymax = static_cast<size_t>(std::max(std::max(nh * hd, kvdim), std::max(H, I)));
@@ -3032,7 +3029,7 @@ bool alloc_prefill(PrefillBufs& pf, const spb_model_config& cfg, int S, std::vec
     // at most one item per split and block of one tile per wave, a partial
     // block more for every sequence
     const size_t tok = kAttnThreads / kWave * 16 / (nh / cfg.num_key_value_heads);
-    pf.max_items = (C / tok + (static_cast<size_t>(nseq) < C ? nseq : C)) * S;
+    pf.max_items = (C / tok + (nseq < C ? nseq : C)) * S;
     return (pf.x = dev_alloc<int8_t>(C * xmax, own)) && (pf.amax = dev_alloc<float>(C, own)) &&
            (pf.y[0] = dev_alloc<int32_t>(C * ystack, own)) &&
            (pf.y[1] = dev_alloc<int32_t>(C * ymax, own)) &&
@@ -3046,7 +3043,27 @@ bool alloc_prefill(PrefillBufs& pf, const spb_model_config& cfg, int S, std::vec
            (pf.pacc = dev_alloc<float>(C * nh * S * hd, own)) &&
            (pf.comb = dev_alloc<float>(C * nh * hd, own)) &&
            (pf.st = dev_alloc<EngineState>(C, own)) &&
-           (tokens > 0 || (pf.items = dev_alloc<PrefillItem>(pf.max_items, own)));
+           (!items || (pf.items = dev_alloc<PrefillItem>(pf.max_items, own)));
+}
+
+// The batched prefill's buffers, for nseq sequences of up to max_seq
+// positions: kPrefillChunk tokens per pass, fewer when the split partials of
+// that many would exceed kPrefillPartialBytes or no prompts have that many, and
+// half as many as long as the device has no room for them (the passes' results
+// do not depend on it).  Called last, so that only this gives way.
+bool alloc_prefill(PrefillBufs& pf, const spb_model_config& cfg, int S, std::vector<void*>& own,
+                   int nseq, int max_seq) {
+    const int nh = cfg.num_attention_heads, hd = cfg.head_dim;
+    const long part = static_cast<long>(nh) * S * (hd + 2) * 4;  // bytes per token
+    long c = std::min<long>(kPrefillPartialBytes / part, kPrefillChunk);
+    c = std::min(c, static_cast<long>(nseq) * (max_seq - 1));  // a prompt's last token is a step's
+    for (c = c > 0 ? c : 1; c > 0; c /= 2) {
+        const size_t held = own.size();
+        if (alloc_pass(pf, cfg, S, own, static_cast<size_t>(c), static_cast<size_t>(nseq), true))
+            return true;
+        for (; own.size() > held; own.pop_back()) (void)hipFree(own.back());
+    }
+    return false;
 }
 
 SegWeights seg_weights(const spb_sparse_linear* a, const spb_sparse_linear* b,
@@ -3828,7 +3845,7 @@ extern "C" int spb_engine_create(const spb_model_config* cfg, const spb_transfor
          (e->rope = dev_alloc<float2>(static_cast<size_t>(max_seq) * (hd / 2), own)) &&
          (e->cur_rope = dev_alloc<float2>(hd / 2, own)) &&
          (e->st = dev_alloc<EngineState>(1, own));
-    ok = ok && alloc_prefill(e->pf, *cfg, e->S, own, 1);
+    ok = ok && alloc_prefill(e->pf, *cfg, e->S, own, 1, max_seq);
     if (!ok) {
         delete e;
         return invalid("%s: device allocation failed", fn);
@@ -4358,8 +4375,7 @@ extern "C" int spb_batch_engine_create(const spb_model_config* cfg,
         ok = e->kcache.back() && e->vcache.back();
     }
     const size_t B = static_cast<size_t>(batch);
-    ok = ok && alloc_prefill(e->step, *cfg, e->S, own, 0, batch) &&
-         alloc_prefill(e->pf, *cfg, e->S, own, batch) &&
+    ok = ok && alloc_pass(e->step, *cfg, e->S, own, B, B, false) &&
          (e->logits = dev_alloc<float>(B * V, own)) &&
          (e->xn = dev_alloc<float>(B * lm_head_batch_xstride(H), own)) &&
          (e->part_lo = dev_alloc<float>(B * e->lm_grid, own)) &&
@@ -4388,6 +4404,7 @@ extern "C" int spb_batch_engine_create(const spb_model_config* cfg,
             ok = ok && (e->gsplit[g].part = dev_alloc<int32_t>(e->split.part_words, own)) &&
                  (e->gsplit[g].count = dev_alloc<unsigned>(kGemmSplitCounters, own));
     }
+    ok = ok && alloc_prefill(e->pf, *cfg, e->S, own, batch, max_seq);
     if (!ok) {
         delete e;
         return invalid("%s: device allocation failed", fn);

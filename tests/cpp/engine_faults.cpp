@@ -5,6 +5,8 @@
 // a launch that fails.
 //   engine_faults launches   every launch of a prompt's generate, and of the
 //                            engines' create, failed once: none may return 0
+//   engine_faults memory     creates on a device with less and less memory: the
+//                            prompts' passes get shorter before create fails
 // Prints one line per check and returns the number of failed ones.
 #include <hip/hip_runtime_api.h>
 
@@ -208,11 +210,44 @@ void launches() {
         check(e.generate(lens) == 0, kind + ": generate afterwards");
     }
 }
+
+void memory() {
+    const Shape s = shape(8, 2, 64, 1024, 2, 4096);
+    for (int batch : {0, 3}) {
+        const std::string kind = batch ? "batch engine" : "engine";
+        const std::vector<int> lens = batch ? std::vector<int>{40, 2100, 1} : std::vector<int>{2100};
+        size_t all = 0;
+        long launched = 0;
+        for (int part = 0; part < 5; ++part) {  // 1, 1/2, ... 1/16 of the memory that create takes
+            g_limit = part ? all >> part : ~size_t{0};
+            Engine e;
+            const int rc = e.create(s, 4096, batch);
+            if (!part) all = g_used;
+            arm(-1);
+            const bool ran = rc == 0 && g_pending == hipSuccess && e.generate(lens) == 0;
+            check(ran && g_launches >= launched,
+                  kind + ": 1/" + std::to_string(1 << part) + " of " + std::to_string(all >> 20) +
+                      " MB, " + std::to_string(g_launches) + " launches");
+            launched = g_launches;
+        }
+        g_limit = 1 << 20;
+        {
+            Engine e;
+            check(e.create(s, 4096, batch) != 0 && g_used == 0 && g_pending == hipSuccess,
+                  kind + ": 1 MB refused, all given back");
+        }
+        g_limit = ~size_t{0};
+        Engine e;  // prompts that cannot fill a pass of 2048 tokens
+        check(e.create(s, 64, batch) == 0 && g_used < all / 16,
+              kind + ": 64 positions take " + std::to_string(g_used >> 20) + " MB");
+    }
+}
 }  // namespace
 
 int main(int argc, char** argv) {
     const std::string what = argc > 1 ? argv[1] : "";
     if (what == "launches") launches();
-    else return std::fprintf(stderr, "usage: %s launches\n", argv[0]), 2;
+    else if (what == "memory") memory();
+    else return std::fprintf(stderr, "usage: %s launches|memory\n", argv[0]), 2;
     return g_bad;
 }

@@ -11,7 +11,7 @@ from tests.conftest import ROOT
 EXE = os.path.join(ROOT, "tests", "cpp", "engine_faults")
 
 
-@pytest.mark.parametrize("what", ["launches"])
+@pytest.mark.parametrize("what", ["launches", "memory"])
 def test_engine_faults(what):
     assert os.path.exists(EXE), "tests/cpp/engine_faults is not built (run __graft_entry__.build())"
     r = subprocess.run([EXE, what], capture_output=True, text=True, timeout=300)
