@@ -290,9 +290,18 @@ long wide_blocks(int rows, int n) {
 // blocks) 53.8 -> 45.7, 104.6 -> 86.6, 147.0 -> 129.6; 6912 x 2560, n = 2048
 // (432) 52.6 -> 46.5; 3840 x 2560, n = 3000 (360) 43.7 -> 43.4, n = 2048 (240)
 // 30.9 -> 31.1; 2560 x 6912, n = 2048 (160) 59.8 -> 65.2.
+//
+// Not so for 17-32 tokens (of 98,000 rows or more): the 64 x 32 tile holds them
+// all and wastes no products.  100352 x 2560, n = 16 / 17 / 32 / 48 / 64 / 65
+// 31.8 -> 29.4, 19.2 -> 29.3, 21.2 -> 31.3, 34.2 -> 33.9, 36.3 -> 36.2, 48.5 ->
+// 36.9; 552960 x 2560, n = 1 / 16 / 32 / 48 145 -> 130, 174 -> 144, 113 -> 153,
+// 200 -> 168; 196608 x 1024, n = 16 / 17 / 32 / 48 55.5 -> 25.1, 17.8 -> 24.5,
+// 18.9 -> 27.1, 32.1 -> 30.8.
 bool wide_ternary_ok(int rows, int cols, int n, const GemmSegs& g) {
-    return 2 * wide_blocks(rows, n) >= 3L * device_cu_count() && cols < (1 << 23) &&
-           (g.end0 >= rows || g.end0 % 16 == 0) && (g.end1 >= rows || g.end1 % 16 == 0);
+    const long blocks = wide_blocks(rows, n), cus = device_cu_count();
+    if (2 * blocks < 3 * cus || (n > 16 && n <= 32)) return false;
+    return cols < (1 << 23) && (g.end0 >= rows || g.end0 % 16 == 0) &&
+           (g.end1 >= rows || g.end1 % 16 == 0);
 }
 
 }  // namespace

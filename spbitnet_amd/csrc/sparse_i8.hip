@@ -286,10 +286,21 @@ void launch_i8_gemm(const uint8_t* comp, const int8_t* B, int32_t* D, int m, int
 
 // The tile for n tokens.  us per launch, the 32 x 64 tile without the loads a
 // step ahead that every size above 16 took before -> now:
-//   * a grid of at least 5/8 wide blocks (256 x 128) per CU: the wide kernel.
-//     13824 x 2560, n = 512 / 1024 / 2048 72.8 -> 31.6, 135 -> 44.2, 263 -> 87.5;
-//     6912 x 2560, n = 1024 / 2048 70.2 -> 32.5, 132 -> 45.5; 2560 x 6912,
-//     n = 2048 (160 blocks) 131 -> 67;
+//   * more than 32 tokens and a grid of at least 5/8 wide blocks (256 x 128)
+//     per CU: the wide kernel.  13824 x 2560, n = 512 / 1024 / 2048 72.8 -> 31.6,
+//     135 -> 44.2, 263 -> 87.5; 6912 x 2560, n = 1024 / 2048 70.2 -> 32.5, 132 ->
+//     45.5; 2560 x 6912, n = 2048 (160 blocks) 131 -> 67.
+//     Up to 32 tokens one block of the tiles below holds them all: the tile that
+//     they choose -> wide, 40960 x 2560 (160 wide blocks), n = 1 / 16 / 17 / 32
+//     10.6 -> 19.6, 11.3 -> 20.5, 12.2 -> 20.8, 13.5 -> 21.9; 100352 x 2560 (392)
+//     23.1 -> 28.6, 24.7 -> 29.8, 26.5 -> 30.0, 28.5 -> 31.6.
+//     The line against the tiles that it displaces: 96 x 32 -> wide, 6912 x
+//     2560, n = 640 / 768 / 896 / 1024 (135 / 162 / 189 / 216 blocks) 25.2 ->
+//     29.9, 28.9 -> 30.4, 32.5 -> 30.8, 36.0 -> 31.4, 4096 x 4096, n = 1024 / 1280
+//     (128 / 160) 54.7 -> 41.3, 65.2 -> 41.9; 128 x 32 -> wide, 2560 x 6912,
+//     n = 1536 / 2048 / 2560 (120 / 160 / 200) 49.4 -> 65.0, 60.8 -> 66.1, 81.0 ->
+//     66.5: for 2560 and 6912 columns it could lie at 190 blocks, for 4096 lower
+//     than it does;
 //   * long rows (over 4096 columns) with at least half a 128 x 32 block per
 //     CU: each activation feeds eight strips; 2560 x 6912, n = 256 / 512 / 1024
 //     27.8 -> 14.9, 41.3 -> 25.6, 78.7 -> 37.4 (54.4 with 96 x 32);
@@ -300,7 +311,7 @@ void launch_i8_gemm(const uint8_t* comp, const int8_t* B, int32_t* D, int m, int
 int launch_i8_for(const uint8_t* comp, const int8_t* B, int32_t* D, int m, int k, int n,
                   hipStream_t st) {
     const long cus = device_cu_count(), passes = (n + 31) / 32;
-    if (8 * wide_blocks(m, n) >= 5 * cus) {
+    if (n > 32 && 8 * wide_blocks(m, n) >= 5 * cus) {
         const WideTiles src{comp, static_cast<int>(i8_strips(m)), static_cast<int>(i8_steps(k))};
         const Int32Out out{D, m, m % 4 == 0 && i8_aligned(D, 16)};
         return launch_wide(src, B, out, m, static_cast<int>(i8_steps(k)), n, k, st);

@@ -1,0 +1,59 @@
+// Which kernel a call launches, by its grid, under the fake runtime of
+// fake_hip.hpp (256 CUs): the lines between the tiles of the sparse GEMMs.
+// Prints one line per check and returns the number of failed ones.
+#include <cstdio>
+#include <vector>
+
+#include "fake_hip.hpp"
+#include "spbitnet_amd.h"
+
+namespace {
+alignas(64) uint32_t g_words[1024];
+int8_t* const g_x = reinterpret_cast<int8_t*>(g_words);
+int32_t* const g_y = reinterpret_cast<int32_t*>(g_words);
+int g_bad = 0;
+
+// One launch whose blocks are tile_rows x tile_tokens.
+void check(const char* what, int rc, int rows, int cols, int n, int tile_rows, int tile_tokens) {
+    const bool ok = rc == 0 && g_launches == 1 &&
+                    static_cast<int>(g_grid.x) == (rows + tile_rows - 1) / tile_rows &&
+                    static_cast<int>(g_grid.y) == (n + tile_tokens - 1) / tile_tokens;
+    std::printf("%s %s %d x %d, n = %d: %ld launches of %u x %u, tiles of %d x %d expected\n",
+                ok ? "ok  " : "FAIL", what, rows, cols, n, g_launches, g_grid.x, g_grid.y,
+                tile_rows, tile_tokens);
+    g_bad += !ok;
+}
+
+void ternary(int rows, int cols, int n, int tile_rows, int tile_tokens) {
+    g_launches = 0;
+    const int rc = spb_sparse_ternary_gemm(g_words, g_words, g_x, g_y, rows, cols, n,
+                                           (cols + 127) / 128 * 4, (cols + 255) / 256 * 4, nullptr);
+    check("ternary", rc, rows, cols, n, tile_rows, tile_tokens);
+}
+
+void sparse_i8(int m, int k, int n, int tile_rows, int tile_tokens) {
+    g_launches = 0;
+    check("int8", spb_sparse_i8_gemm(g_words, g_x, g_y, m, k, n, nullptr), m, k, n, tile_rows,
+          tile_tokens);
+}
+}  // namespace
+
+int main() {
+    // the wide kernel from 384 blocks on
+    ternary(6144, 2560, 2048, 256, 128);
+    ternary(5888, 2560, 2048, 128, 64);
+    // few tokens of many rows
+    ternary(98304, 2560, 16, 256, 128);
+    ternary(98304, 2560, 17, 64, 32);
+    ternary(552960, 2560, 32, 64, 32);
+    ternary(98304, 2560, 33, 256, 128);
+    sparse_i8(40960, 2560, 1, 32, 16);
+    sparse_i8(40960, 2560, 16, 32, 16);
+    sparse_i8(40960, 2560, 32, 64, 32);
+    sparse_i8(100352, 2560, 32, 96, 32);
+    sparse_i8(41984, 6912, 32, 128, 32);
+    sparse_i8(40960, 2560, 33, 256, 128);
+    sparse_i8(6912, 2560, 768, 256, 128);
+    sparse_i8(6912, 2560, 640, 96, 32);
+    return g_bad;
+}

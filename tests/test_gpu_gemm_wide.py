@@ -30,7 +30,10 @@ def _tokens(n, cols, seed):
 
 # at least 384 blocks each (1.5 per CU); cols / 128 = 2, 4, 6, 10 steps
 @pytest.mark.parametrize("rows,cols,n", [(4096, 256, 3072), (4001, 512, 3073), (8190, 768, 1601),
-                                         (257, 1280, 25000), (100000, 256, 1), (13825, 1280, 1000)])
+                                         (257, 1280, 25000), (100000, 256, 1), (13825, 1280, 1000),
+                                         # beside the lines to the staged tiles
+                                         (100000, 256, 16), (100000, 256, 17), (100000, 256, 32),
+                                         (100000, 256, 33)])
 def test_ternary_wide(gpu, rows, cols, n):
     L, meta, values, dense = _ternary(rows, cols, rows + n)
     X = _tokens(n, cols, n)
@@ -46,7 +49,8 @@ def test_ternary_wide(gpu, rows, cols, n):
 
 
 @pytest.mark.parametrize("m,k,n", [
-    (4097, 144, 1600), (6000, 272, 1025), (49200, 64, 3),     # wide: 160 blocks or more
+    (4097, 144, 1600), (6000, 272, 1025), (49200, 64, 33),    # wide: 160 blocks or more
+    (49200, 64, 3), (40970, 272, 17), (49170, 64, 32),        # as many, up to 32 tokens
     (6912, 400, 230), (97, 2560, 5500),                       # 96 x 32: 512 blocks or more
     (2560, 4112, 201), (129, 6912, 2100),                     # long rows: 128 x 32
     (640, 48, 17), (33, 2560, 40), (2560, 4096, 33), (50, 6912, 64),  # 64 x 32
