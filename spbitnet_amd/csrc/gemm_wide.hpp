@@ -291,15 +291,26 @@ long wide_blocks(int rows, int n) {
 // (432) 52.6 -> 46.5; 3840 x 2560, n = 3000 (360) 43.7 -> 43.4, n = 2048 (240)
 // 30.9 -> 31.1; 2560 x 6912, n = 2048 (160) 59.8 -> 65.2.
 //
-// Not so for 17-32 tokens (of 98,000 rows or more): the 64 x 32 tile holds them
-// all and wastes no products.  100352 x 2560, n = 16 / 17 / 32 / 48 / 64 / 65
-// 31.8 -> 29.4, 19.2 -> 29.3, 21.2 -> 31.3, 34.2 -> 33.9, 36.3 -> 36.2, 48.5 ->
-// 36.9; 552960 x 2560, n = 1 / 16 / 32 / 48 145 -> 130, 174 -> 144, 113 -> 153,
-// 200 -> 168; 196608 x 1024, n = 16 / 17 / 32 / 48 55.5 -> 25.1, 17.8 -> 24.5,
-// 18.9 -> 27.1, 32.1 -> 30.8.
+// Not so in two places (same runs, staged -> wide):
+//   * 17-32 tokens of 98,000 rows or more: the 64 x 32 tile holds them all and
+//     wastes no products.  100352 x 2560, n = 16 / 17 / 32 / 48 / 64 / 65 31.8
+//     -> 29.4, 19.2 -> 29.3, 21.2 -> 31.3, 34.2 -> 33.9, 36.3 -> 36.2, 48.5 ->
+//     36.9; 552960 x 2560, n = 1 / 16 / 32 / 48 145 -> 130, 174 -> 144, 113 ->
+//     153, 200 -> 168; 196608 x 1024, n = 16 / 17 / 32 / 48 55.5 -> 25.1, 17.8
+//     -> 24.5, 18.9 -> 27.1, 32.1 -> 30.8.
+//   * The first quarter of a third block per CU (513-576 blocks): a few CUs run
+//     three.  2048 tokens, 8448 rows (528) at 512 / 1024 / 1536 / 2048 / 2560 /
+//     4096 / 5120 / 6912 columns 26.0 -> 27.6, 34.2 -> 38.7, 44.5 -> 48.4, 58.6
+//     -> 61.7, 66.2 -> 67.7, 95.1 -> 100, 113 -> 120, 156.4 -> 156.6; 9216 rows
+//     (576) at 1024 / 2560 / 4096 / 6912 35.8 -> 38.8, 65.9 -> 64.4, 93.3 ->
+//     97.3, 154 -> 146; 9472 (592) at 1024 / 2560 / 4096 37.9 -> 38.7, 71.6 ->
+//     68.6, 104.5 -> 101.0.  Past a third and a fourth block the wide kernel
+//     wins but for 1024-1536 columns, within 3 % (784 blocks at 1024 48.5 ->
+//     50.0).
 bool wide_ternary_ok(int rows, int cols, int n, const GemmSegs& g) {
     const long blocks = wide_blocks(rows, n), cus = device_cu_count();
     if (2 * blocks < 3 * cus || (n > 16 && n <= 32)) return false;
+    if (blocks > 2 * cus && 4 * blocks <= 9 * cus && cols <= 5120) return false;
     return cols < (1 << 23) && (g.end0 >= rows || g.end0 % 16 == 0) &&
            (g.end1 >= rows || g.end1 % 16 == 0);
 }

@@ -47,6 +47,12 @@ int main() {
     ternary(98304, 2560, 17, 64, 32);
     ternary(552960, 2560, 32, 64, 32);
     ternary(98304, 2560, 33, 256, 128);
+    // a little past two blocks per CU
+    ternary(8192, 1024, 2048, 256, 128);
+    ternary(8193, 1024, 2048, 128, 64);
+    ternary(9216, 5120, 2048, 128, 64);
+    ternary(9217, 1024, 2048, 256, 128);
+    ternary(8448, 5376, 2048, 256, 128);
     sparse_i8(40960, 2560, 1, 32, 16);
     sparse_i8(40960, 2560, 16, 32, 16);
     sparse_i8(40960, 2560, 32, 64, 32);

@@ -33,7 +33,7 @@ def _tokens(n, cols, seed):
                                          (257, 1280, 25000), (100000, 256, 1), (13825, 1280, 1000),
                                          # beside the lines to the staged tiles
                                          (100000, 256, 16), (100000, 256, 17), (100000, 256, 32),
-                                         (100000, 256, 33)])
+                                         (100000, 256, 33), (8193, 256, 2047), (9217, 256, 2047)])
 def test_ternary_wide(gpu, rows, cols, n):
     L, meta, values, dense = _ternary(rows, cols, rows + n)
     X = _tokens(n, cols, n)
