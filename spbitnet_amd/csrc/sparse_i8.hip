@@ -162,26 +162,35 @@ __global__ __launch_bounds__(W * kWave) void sparse_i8_gemm_kernel(
     for (int s = 0; s < S; ++s)
 #pragma unroll
         for (int t = 0; t < T; ++t) acc[s][t] = (v4i){0, 0, 0, 0};
-    // a step's operands, loaded one step ahead of their products: strips past
-    // the matrix read its last one (their rows are not stored), and the loads
-    // past a wave's last step read a step again
+    // a step's operands, loaded one step ahead of their products; strips past
+    // the matrix read its last one (their rows are not stored), and loads past
+    // a wave's last step get empty extents: zeros, without a trip to memory.
+    // Reading a step again there cost short rows most, us: 13824 x 1024, n = 128
+    // / 256 9.7 -> 8.9, 14.4 -> 12.7; 30000 x 1024, n = 1 / 8 / 16 3.6 -> 3.6, 4.6
+    // -> 4.4, 5.8 -> 5.2 (3.4, 4.1 and 4.9 without loads ahead, which
+    // everywhere else are the faster form: 6912 x 6912, n = 16 8.1 -> 6.7).
     struct Step {
         v4i a[S];
         int idx[S];
         v4i lo[T], hi[T];
     };
     auto load = [&](int j, Step& o) {
-        j = j < steps ? j : steps - 1;
+        const bool live = j < steps;  // uniform
 #pragma unroll
         for (int s = 0; s < S; ++s) {
             const int strip = s0 + s < strips ? s0 + s : strips - 1;
-            const uint8_t* tp = comp + (static_cast<long>(strip) * steps + j) * kI8TileBytes;
-            o.a[s] = *reinterpret_cast<const v4i*>(tp + lane * 16);
-            o.idx[s] = *reinterpret_cast<const int*>(tp + kI8ValBytes + lane * 4);
+            const __amdgpu_buffer_rsrc_t ra = __builtin_amdgcn_make_buffer_rsrc(
+                const_cast<uint8_t*>(comp + (static_cast<long>(strip) * steps + (live ? j : 0)) *
+                                                kI8TileBytes),
+                static_cast<short>(0), live ? kI8TileBytes : 0, kI8RawBufferFlags);
+            o.a[s] = __builtin_bit_cast(
+                v4i, __builtin_amdgcn_raw_buffer_load_b128(ra, lane * 16, 0, 0));
+            o.idx[s] = static_cast<int>(
+                __builtin_amdgcn_raw_buffer_load_b32(ra, kI8ValBytes + lane * 4, 0, 0));
         }
 #pragma unroll
         for (int t = 0; t < T; ++t) {
-            const int off = (t0 + 16 * t + li) * k + 128 * j + 16 * q;
+            const int off = live ? (t0 + 16 * t + li) * k + 128 * j + 16 * q : n * k;
             o.lo[t] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(rb, off, 0, 0));
             o.hi[t] =
                 __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(rb, off + 64, 0, 0));
