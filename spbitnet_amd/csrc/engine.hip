@@ -3272,12 +3272,20 @@ void launch_attn_combine(int hd, int nh, int splits, hipStream_t s, const float*
 // attention's first `splits` splits: the split combine over (head, token),
 // then one block per token; with few splits the token's block folds them
 // itself (the same operations in the same order), a launch and a trip through
-// memory less.
+// memory less.  Few: up to 4, and up to 8 where a token's heads are at most
+// kFoldLongCols wide (wider ones have too many loads for one block).  Decode
+// steps of 6 layers, us, apart -> folded: 2560 wide, 2 / 32 / 128 sequences at
+// position 60 313 -> 304, 378 -> 368, 570 -> 557, at 450 317 -> 316, 427 -> 423,
+// 697 -> 692; 4096 wide at 200 394 -> 387, 522 -> 513, 765 -> 755, at 300 395 ->
+// 401, 548 -> 556, 836 -> 844.  Prompts through 4 layers: 4096 wide, 200 / 300 /
+// 500 tokens 656 -> 649, 767 -> 774, 936 -> 950; 8192 wide, 200 / 400 / 500 941 ->
+// 934, 1341 -> 1360, 1519 -> 1543.
+constexpr int kFoldLongCols = 3072;
 void launch_attn_input(int hd, int nh, int splits, hipStream_t s, const float* pm,
                        const float* pl, const float* pacc, float* comb, const EngineState* st,
                        int S, int B, int8_t* x, float* amax) {
     const int n = nh * hd;
-    if (splits <= kFusedCombineSplits) {
+    if (splits <= (n <= kFoldLongCols ? kFusedCombineSplits : kFusedCombineSplits / 2)) {
         const AttnCombine p{pm, pl, pacc, hd, S, n, hd == 64 ? 6 : 7};
         launch_prefill_producer(p, n, st, n, B, x, amax, s);
         return;

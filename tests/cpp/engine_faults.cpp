@@ -4,6 +4,8 @@
 //                            engines' create, failed once: none may return 0
 //   engine_faults memory     creates on a device with less and less memory: the
 //                            prompts' passes get shorter before create fails
+//   engine_faults folds      launches of a prompt: one less per layer where the
+//                            o projection's producer folds the splits itself
 // Prints one line per check and returns the number of failed ones.
 #include <cstdio>
 #include <string>
@@ -146,12 +148,35 @@ void memory() {
               kind + ": 64 positions take " + std::to_string(g_used >> 20) + " MB");
     }
 }
+
+void folds() {
+    // prompts of 1-4, 5-8 and more splits, heads of a token 1024 and 4096 wide
+    const bool narrow[3] = {true, true, false}, wide[3] = {true, false, false};
+    for (int heads : {8, 32}) {
+        const Shape s = shape(heads, 8, 128, 1024, 2, 1024);
+        Engine e;
+        check(e.create(s, 1024, 0) == 0, "create");
+        long most = 0, got[3];
+        for (int k : {2, 1, 0}) {
+            const int tokens[3] = {257, 513, 514};  // the last is a step's
+            arm(-1);
+            check(e.generate({tokens[k]}) == 0, "generate");
+            got[k] = g_launches;
+            most = got[k] > most ? got[k] : most;
+        }
+        for (int k = 0; k < 3; ++k)
+            check(got[k] == most - ((heads == 8 ? narrow : wide)[k] ? 2 : 0),
+                  std::to_string(128 * heads) + " wide, prompt " + std::to_string(k) + ": " +
+                      std::to_string(got[k]) + " launches of " + std::to_string(most));
+    }
+}
 }  // namespace
 
 int main(int argc, char** argv) {
     const std::string what = argc > 1 ? argv[1] : "";
     if (what == "launches") launches();
     else if (what == "memory") memory();
-    else return std::fprintf(stderr, "usage: %s launches|memory\n", argv[0]), 2;
+    else if (what == "folds") folds();
+    else return std::fprintf(stderr, "usage: %s launches|memory|folds\n", argv[0]), 2;
     return g_bad;
 }
