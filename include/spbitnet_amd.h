@@ -107,9 +107,10 @@ int spb_dequantize_bf16(const int32_t* input, uint16_t* output, const float* d_a
  * absmax_reduce_gpu into the engine's d_absmax_ scratch, then
  * fused_sparse_bitlinear_gpu) as one call; the scratch comes in as a caller
  * workspace of at least spb_bitlinear_workspace_size(cols) bytes, 16-byte
- * aligned (the absmax, then the quantised activations as bit planes, built
- * once instead of in every GEMV workgroup when cols % 8 == 0 and x is 16-byte
- * aligned).  Output bits equal the reference pair's:
+ * aligned.  After the call it holds the absmax (a float, at byte 0) and, when
+ * cols % 8 == 0 and x is 16-byte aligned, the quantised activations as bit
+ * planes (at byte 256, the layout of spb_absmax_quantize_planes_*).  Output
+ * bits equal the reference pair's:
  * output[r] = 16-bit(float(W q) * ((gamma * absmax) / 127)),
  * q = clamp(rint(x * (absmax > 0 ? 127/absmax : 0)), -128, 127).
  * Calls that share a workspace must be ordered (same stream). */

@@ -8,8 +8,9 @@
 //                             spb_absmax_quantize_planes_*)
 // One launch where every block's rows are a few steps of the span kernel (the
 // decode shapes: cols % 128 == 0, up to 8192, and ~25,000 rows at 2560 columns):
-// each block quantises the vector for itself while its weights arrive.  bf16
-// 2560 x 6912: 3.7 + 4.4 us in two launches before, 4.7 us now.
+// each block quantises the vector for itself while its weights arrive, and one
+// writes the workspace.  bf16 2560 x 6912: 3.7 + 4.4 us in two launches before,
+// 4.7 us now.
 // Else, when cols % 8 == 0 and x and the workspace are 16-byte aligned, the
 // planes are built once (spb_absmax_quantize_planes_*, one block) and the GEMV reads
 // them (spb_fused_sparse_bitlinear_planes_*), instead of every GEMV block
@@ -50,14 +51,17 @@ bool overlap(const void* a, size_t na, const void* b, size_t nb) {
 template <class T>
 bool bitlinear_span(const uint32_t* meta, const uint32_t* values, const uint16_t* x,
                     uint16_t* output, float gamma, int rows, int cols, int ms, int vs,
-                    hipStream_t s) {
-    if (!bitplane_ok(meta, values, cols, ms, vs) || !aligned(x, 16) || cols > 16 * kBlock ||
+                    float* d_absmax, uint32_t* planes, hipStream_t s) {
+    if (!bitplane_ok(meta, values, cols, ms, vs) || !aligned(x, 16) || !aligned(planes, 16) ||
+        cols > 16 * kBlock ||
         overlap(x, 2 * static_cast<size_t>(cols), output, 2 * static_cast<size_t>(rows)))
         return false;
     const Weights wt{meta, values, rows, cols, ms, vs};
     const DequantOwnSink<T> sink{output, gamma, 0.0f};
-    if (cols <= 8 * kBlock) return launch_span(wt, AbsmaxPlanes<T, 1>{x, cols / 8, 0.0f}, sink, s);
-    return launch_span(wt, AbsmaxPlanes<T, 2>{x, cols / 8, 0.0f}, sink, s);
+    uint4* const p = reinterpret_cast<uint4*>(planes);
+    if (cols <= 8 * kBlock)
+        return launch_span(wt, AbsmaxPlanes<T, 1>{x, cols / 8, d_absmax, p, 0.0f}, sink, s);
+    return launch_span(wt, AbsmaxPlanes<T, 2>{x, cols / 8, d_absmax, p, 0.0f}, sink, s);
 }
 
 // The BitLinear on a workspace already checked to hold workspace_bytes(cols).
@@ -69,7 +73,7 @@ int bitlinear_ws(const char* fn, const uint32_t* meta, const uint32_t* values, c
     uint32_t* planes = reinterpret_cast<uint32_t*>(ws + kAbsmaxBytes);
     constexpr bool kBf16 = std::is_same<T, BF16>::value;
     int rc;
-    if (bitlinear_span<T>(meta, values, x, output, gamma, rows, cols, ms, vs, s)) {
+    if (bitlinear_span<T>(meta, values, x, output, gamma, rows, cols, ms, vs, d_absmax, planes, s)) {
         rc = launch_status(fn);
         if (rc) return rc;
     } else if (cols % 8 == 0 && aligned(x, 16) && aligned(ws, 16)) {

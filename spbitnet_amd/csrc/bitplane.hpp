@@ -353,11 +353,15 @@ struct GlobalPlanes {
 // Planes of 16-bit activations that the block itself quantises with their own
 // absmax (the whole BitLinear in one launch): at most KU 16-byte units per
 // thread, loaded ahead of the weights and kept in registers through the
-// absmax.  The rule and the absmax are QuantSrc's and block_absmax's.
+// absmax.  The rule and the absmax are QuantSrc's and block_absmax's.  One
+// block leaves the absmax and the planes in memory as
+// spb_absmax_quantize_planes_* does, for a caller that reads them.
 template <class T, int KU>
 struct AbsmaxPlanes {
     const uint16_t* x;
     int units;  // cols / 8 <= KU * kBlock
+    float* out_amax;
+    uint4* out_planes;  // word w of planes 4 h .. 4 h + 3 at [2 w + h]
     float amax;
     struct Regs {
         uint4 r[KU];
@@ -405,6 +409,22 @@ struct AbsmaxPlanes {
             }
         }
     }
+    __device__ void publish(const uint32_t* planes, int nw, int tid) const {
+        for (int i = tid; i < 2 * nw; i += kBlock) {
+            const uint32_t* p = planes + 4 * (i & 1) * nw + (i >> 1);
+            out_planes[i] = make_uint4(p[0], p[nw], p[2 * nw], p[3 * nw]);
+        }
+        if (tid == 0) *out_amax = amax;
+    }
+};
+// Activations whose last block publishes them once its planes are built.
+template <class Act>
+struct ActPublishes {
+    static constexpr bool value = false;
+};
+template <class T, int KU>
+struct ActPublishes<AbsmaxPlanes<T, KU>> {
+    static constexpr bool value = true;
 };
 
 // ---- output sinks ------------------------------------------------------------------
@@ -697,6 +717,8 @@ __global__ __launch_bounds__(kBlock) void gemv_span_kernel(W wt, Act act, Sink s
     for (int i = tid; i < MS * RS; i += kBlock) acc[i] = 0;
     __syncthreads();
     sink.bind(act);
+    if constexpr (ActPublishes<Act>::value)
+        if (blockIdx.x == gridDim.x - 1) act.publish(planes, nwords, tid);
     if (ro < RS) {
         load_x(planes, c, nwords, X);
 #pragma unroll

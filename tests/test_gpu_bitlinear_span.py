@@ -59,6 +59,24 @@ def test_one_launch_equals_the_pair(gpu, kind, rows, cols):
         assert (same | (got.isnan() & want.isnan())).all(), name
 
 
+@pytest.mark.parametrize("kind", ["f16", "bf16"])
+@pytest.mark.parametrize("rows,cols", [(1, 128), (257, 384), (25600, 2560), (513, 4224),
+                                       (100, 8192), (70, 8320), (25601, 2560), (33, 1000)])
+def test_workspace_holds_absmax_and_planes(gpu, kind, rows, cols):
+    """The workspace afterwards: the absmax, and from byte 256 on the planes of
+    absmax_quantize_planes_gpu, in one launch (to 8192 columns) as in two."""
+    meta, values, L = _layer(rows, cols // 64 * 64 + (64 if cols % 64 else 0))
+    x = torch.randn(cols, device="cuda").to(HALF[kind])
+    planes = torch.empty(8 * -(-cols // 32), dtype=torch.int32, device="cuda")
+    amax = torch.empty(1, dtype=torch.float32, device="cuda")
+    K.absmax_quantize_planes_gpu(x, planes, amax, cols)
+    ws = torch.full((K.bitlinear_workspace_size(cols),), 0xA5, dtype=torch.uint8, device="cuda")
+    out = torch.empty(rows, dtype=x.dtype, device="cuda")
+    K.bitlinear_gpu(meta, values, x, out, L.gamma, rows, cols, L.meta_stride, L.values_stride, ws)
+    assert torch.equal(ws[:4].view(torch.float32), amax)
+    assert torch.equal(ws[256:].view(torch.int32), planes)
+
+
 def test_output_over_input(gpu):
     meta, values, L = _layer(2560, 2560)
     x = torch.randn(2560, device="cuda").to(torch.bfloat16)
