@@ -23,6 +23,25 @@ def _ternary(rows, cols, seed):
     return L, meta, values, dense
 
 
+@pytest.mark.parametrize("nh,nkv,ffn", [(26, 13, 3200), (48, 12, 1024)])
+def test_wide_stacks_in_an_engine(gpu, nh, nkv, ffn):
+    """Passes of 2048 prompt tokens whose projections take the wide kernel, against
+    one decode step per token, bit for bit: 26 heads: q | k | v (boundaries at rows
+    3328 and 4992, the latter inside a 256-row block) and gate | up (3200, inside a
+    block) with the bf16 sink; 48 heads: o and down with the bf16 and residual sinks."""
+    from spbitnet_amd.model import Model, ModelConfig
+    from tests.test_gpu_engine import _prompt
+    from tests.test_gpu_prefill_attention import _both
+    cfg = ModelConfig(hidden_size=128 * nh, num_hidden_layers=1, num_attention_heads=nh,
+                      num_key_value_heads=nkv, intermediate_size=ffn, vocab_size=512,
+                      max_position_embeddings=2100, head_dim=128)
+    model = Model.random(cfg, seed=nh)
+    print(f"hidden {cfg.hidden_size}", flush=True)
+    batched, stepwise = _both(model, 2100, _prompt(2049, cfg.vocab_size, nh))
+    assert torch.isfinite(stepwise).all()
+    assert torch.equal(batched.view(torch.int32), stepwise.view(torch.int32))
+
+
 def _tokens(n, cols, seed):
     g = torch.Generator(device="cuda").manual_seed(seed)
     return torch.randint(-128, 128, (n, cols), dtype=torch.int8, device="cuda", generator=g)
