@@ -444,6 +444,10 @@ int spb_engine_set_prefill_batch(spb_engine* engine, int min_tokens);
 int spb_engine_decode_steps(spb_engine* engine, int steps);
 /* Device buffers: logits float32 [vocab], tokens int32 [max_seq + 1]. */
 int spb_engine_buffers(const spb_engine* engine, const float** logits, const int** tokens);
+/* A layer's caches on the device, bf16 [num_key_value_heads][max_seq]
+ * [head_dim], K after RoPE: to read (positions below spb_engine_seq_len). */
+int spb_engine_kv_cache(const spb_engine* engine, int layer, const uint16_t** k,
+                        const uint16_t** v);
 
 /* ---- batched decode engine --------------------------------------------------
  * No reference counterpart: the reference decodes one sequence per engine

@@ -4048,6 +4048,18 @@ extern "C" int spb_engine_buffers(const spb_engine* e, const float** logits, con
     return 0;
 }
 
+extern "C" int spb_engine_kv_cache(const spb_engine* e, int layer, const uint16_t** k,
+                                   const uint16_t** v) {
+    clear_error();
+    const char* fn = "spb_engine_kv_cache";
+    if (!e || !k || !v) return invalid("%s: null argument", fn);
+    if (layer < 0 || layer >= e->cfg.num_hidden_layers)
+        return invalid("%s: layer %d outside [0, %d)", fn, layer, e->cfg.num_hidden_layers);
+    *k = e->kcache[layer];
+    *v = e->vcache[layer];
+    return 0;
+}
+
 extern "C" int spb_generate_sparse_ternary(uint64_t seed, int rows, int cols, uint32_t* meta,
                                            uint32_t* values, int meta_stride, int values_stride,
                                            float* d_gamma, float* latent, spb_stream_t stream) {

@@ -487,6 +487,23 @@ class InferenceEngine:
         _lib.check(self._L.spb_engine_decode_steps(self._h, int(steps)),
                    "spb_engine_decode_steps")
 
+    def kv_cache(self, layer: int) -> tuple:
+        """Copies of a layer's K (after RoPE) and V cache, bf16
+        [kv heads][max_seq][head_dim]."""
+        kp, vp = ctypes.c_void_p(), ctypes.c_void_p()
+        _lib.check(self._L.spb_engine_kv_cache(self._h, int(layer), ctypes.byref(kp),
+                                               ctypes.byref(vp)), "spb_engine_kv_cache")
+        c = self.model.config
+        out = []
+        torch.cuda.synchronize()
+        for p in (kp, vp):
+            t = torch.empty((c.num_key_value_heads, self.max_seq, c.head_dim),
+                            dtype=torch.bfloat16, device=self._logits.device)
+            _lib.memcpy_d2d(t.data_ptr(), p.value, t.numel() * 2, None)
+            out.append(t)
+        torch.cuda.synchronize()
+        return tuple(out)
+
 
 class BatchInferenceEngine:
     """Greedy decode of several independent sequences per step on the HIP

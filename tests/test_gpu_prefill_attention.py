@@ -1,7 +1,8 @@
 """The prefill attention on the float32 matrix cores against the decode step:
 a prompt prefilled in batches leaves the same logits, bit for bit, as one
 decode step per token, at the edges of its tiles (16 rows of token x head, 64
-positions, blocks of several tiles) and with values of V that are not finite."""
+positions, blocks of several tiles) and with positions of K or V that are not
+finite."""
 import pytest
 import torch
 
@@ -42,22 +43,61 @@ def test_prefill_attention_tile_edges(gpu, hd, nkv):
         assert torch.equal(batched.view(torch.int32), stepwise.view(torch.int32)), n
 
 
+def _dense_row(lin, row):
+    """Row `row` of a packed matrix as {-1, 0, 1} floats."""
+    from spbitnet_amd import kernels as K
+    dense = torch.empty((lin.rows, lin.cols), dtype=torch.int8, device="cuda")
+    K.sparse_ternary_unpack_gpu(lin.meta, lin.values, dense, lin.rows, lin.cols, lin.meta_stride,
+                                lin.values_stride)
+    return dense[row].float()
+
+
+@pytest.mark.parametrize("which", ["v", "k"])
 @pytest.mark.parametrize("hd,nkv", [(64, 1), (128, 2)])
-def test_prefill_attention_non_finite_values(gpu, hd, nkv):
-    """An infinite V at a later position leaves earlier tokens alone (its
-    weight is not 0 times infinity: the position is not theirs to see)."""
-    from spbitnet_amd.model import Model
+def test_prefill_attention_non_finite_positions(gpu, hd, nkv, which):
+    """A position whose V (or K) is infinite leaves the tokens before it alone:
+    it is not theirs to see, and a weight of 0 times infinity would be NaN.  The
+    first layer's attention of those tokens shows in the second layer's K and V
+    rows, which have to be finite and those of one decode step per token, bit for
+    bit.  One token's embedding is a row of the projection, so that its product is
+    some 20 times the others' spread and it alone passes the largest float."""
+    from spbitnet_amd.model import InferenceEngine, Model
     cfg = _small_config(num_key_value_heads=nkv, head_dim=hd, hidden_size=8 * hd)
     model = Model.random(cfg, seed=hd + nkv)
+    first, H = model.layers[0], cfg.hidden_size
     for lin in ("q_proj", "k_proj"):
         for l in model.layers:
             getattr(l, lin).gamma *= 0.05
-    # products reach about 3000 (4 sigma over 512 or 1024 columns): the largest overflow
-    model.layers[0].v_proj.gamma = 3e38 / 2000 * 127 / 4
-    for n in (40, 100):
-        batched, stepwise = _both(model, 256, _prompt(n, cfg.vocab_size, n))
-        same = batched.view(torch.int32) == stepwise.view(torch.int32)
-        assert (same | (batched.isnan() & stepwise.isnan())).all()
+    big = 7  # the token
+    lin = first.v_proj if which == "v" else first.k_proj
+    model.embed_tokens[big] = 0.02 * _dense_row(lin, 0).to(torch.bfloat16)
+    first.input_layernorm.fill_(1.0)
+    # the token's row is H / 2 values of sqrt(2), all quantised to 127: its product
+    # is gamma * H / 2 * sqrt(2), 1.1 times the largest float
+    lin.gamma = 1.1 * 3.4e38 / (H / 2 * 2 ** 0.5)
+    if which == "v":
+        first.o_proj.gamma *= 1e-37  # outputs of the usual size
+    else:
+        first.q_proj.gamma *= 1e-36  # scores of a few units
+    eng = InferenceEngine(model, max_seq=256)
+    # the only split of the prompt; its second split, of 36 positions; its third
+    for at, n in ((21, 40), (70, 100), (150, 170)):
+        prompt = [t if t != big else 8 for t in _prompt(n, cfg.vocab_size, n)]
+        prompt[at] = big
+        rows, logits = [], []
+        for batch in (1, 0):
+            eng.set_prefill_batch(batch)
+            eng.generate(prompt, 1, stop_at_eos=False)
+            logits.append(_last_logits(eng))
+            k0, v0 = eng.kv_cache(0)
+            assert not (v0 if which == "v" else k0)[:, at].isfinite().all()
+            assert (v0 if which == "v" else k0)[:, :at].isfinite().all()
+            rows.append(torch.cat([c[:, :at] for c in (k0, v0, *eng.kv_cache(1))]))
+        assert rows[1].isfinite().all(), (at, n)
+        assert torch.equal(rows[0].view(torch.int16), rows[1].view(torch.int16)), (at, n)
+        same = logits[0].view(torch.int32) == logits[1].view(torch.int32)
+        assert (same | (logits[0].isnan() & logits[1].isnan())).all()
+    eng.close()
 
 
 @pytest.mark.parametrize("hd,nkv", [(64, 4), (128, 1)])
