@@ -257,7 +257,7 @@ def test_engine_batched_prefill_matches_stepwise(gpu):
     step are bit-identical and the generated tokens equal; prompts that span
     several prefill passes and attention splits, GQA groups 8, 4 and 1, head
     dims 64 and 128, with and without sub-norms."""
-    # 2100 tokens: three prefill passes (1024, 1024, 51 tokens) and 33 splits
+    # 2100 tokens: two prefill passes (2048 and 51 tokens) and 33 splits
     hd128 = dict(head_dim=128, hidden_size=1024)
     cases = [({}, dict(), 2, 2200, 2100), ({}, dict(sub_norms=False), 2, 96, 40),
              ({}, dict(), 8, 320, 300), ({}, dict(), 1, 64, 17), (hd128, dict(), 2, 200, 150),

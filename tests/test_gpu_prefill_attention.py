@@ -3,9 +3,13 @@ a prompt prefilled in batches leaves the same logits, bit for bit, as one
 decode step per token, at the edges of its tiles (16 rows of token x head, 64
 positions, blocks of several tiles) and with positions of K or V that are not
 finite."""
+import os
+import subprocess
+
 import pytest
 import torch
 
+from tests.conftest import ROOT
 from tests.test_gpu_engine import _last_logits, _prompt, _small_config
 
 pytestmark = pytest.mark.gpu
@@ -41,6 +45,40 @@ def test_prefill_attention_tile_edges(gpu, hd, nkv):
         batched, stepwise = _both(model, 768, _prompt(n, cfg.vocab_size, n))
         assert torch.isfinite(stepwise).all()
         assert torch.equal(batched.view(torch.int32), stepwise.view(torch.int32)), n
+
+
+@pytest.mark.parametrize("max_seq,n", [(4300, 4150), (262144, 800)])
+def test_prefill_attention_three_passes(gpu, max_seq, n):
+    """Passes that start past the prompt's first: 2048 + 2048 + 53 tokens, and four
+    of at most 248, as many as 4096 splits' partials leave below 2 GB (which also
+    takes the split combine that has no room for the weights of all splits)."""
+    from spbitnet_amd.model import InferenceEngine, Model
+    cfg = _small_config(max_position_embeddings=max_seq, num_key_value_heads=1)
+    model = Model.random(cfg, seed=n)
+    for lin in ("q_proj", "k_proj"):
+        for l in model.layers:
+            getattr(l, lin).gamma *= 0.05
+    eng = InferenceEngine(model, max_seq=max_seq)
+    out = []
+    for batch in (1, 0):
+        eng.set_prefill_batch(batch)
+        eng.generate(_prompt(n, cfg.vocab_size, n), 1, stop_at_eos=False)
+        out.append([_last_logits(eng)] + [c[:, :n].clone() for c in eng.kv_cache(1)])
+        print(f"max_seq={max_seq} n={n} batch={batch}", flush=True)
+    eng.close()
+    assert torch.isfinite(out[1][0]).all()
+    for got, want in zip(*out):
+        assert torch.equal(got, want)
+
+
+def test_mfma_is_a_chain_of_fused_multiply_adds(gpu):
+    """What the kernel's equality rests on (tests/cpp/mfma_chain.hip, built by
+    __graft_entry__.build())."""
+    exe = os.path.join(ROOT, "tests", "cpp", "mfma_chain")
+    assert os.path.exists(exe), "tests/cpp/mfma_chain is not built"
+    r = subprocess.run([exe], capture_output=True, text=True, timeout=100)
+    print(r.stdout, flush=True)
+    assert r.returncode == 0, r.stdout + r.stderr
 
 
 def _dense_row(lin, row):
