@@ -10,6 +10,8 @@
 // 1/sqrt is correctly rounded where the reference uses rsqrtf, and reductions
 // use wave-64 trees.  Shapes are validated on the host; every kernel bounds-
 // checks its own indices.
+#include <algorithm>
+
 #include "common.hpp"
 #include "spbitnet_amd.h"
 
@@ -148,22 +150,23 @@ __device__ __forceinline__ int first_head(int k, int nh, int nkv) {
 }
 
 // The same scores for head_dim 8 L, L = 4, 8, 16 or 32, and 16-byte aligned
-// rows: L lanes take a K row, 16 bytes each, once for all q heads of its kv
-// head.  A launch is one round trip per block: the kernel above reads 2 bytes
-// per lane and every K row once per q head (20 heads on 5, head_dim 128, 2500
-// positions: 9.2 us, 3.5 us with this one).
+// rows: L lanes take a K row, 16 bytes each, once for `per` q heads of its kv
+// head (blockIdx.z: which).  A launch is one round trip per block: the kernel
+// above reads 2 bytes per lane and every K row once per q head (20 heads on 5,
+// head_dim 128, 2500 positions: 9.2 us, 3.5 us with this one).
 template <class T, int L>
 __global__ __launch_bounds__(kOpBlock) void attention_scores_rows_kernel(
     const uint16_t* Q, const uint16_t* K, float* scores, int nh, int nkv, int max_seq,
-    int seq_len, float scale) {
+    int seq_len, float scale, int per) {
     const int c = threadIdx.x % L, kvh = blockIdx.y;
     const int j = blockIdx.x * (kOpBlock / L) + threadIdx.x / L;
     const int jr = j < seq_len ? j : seq_len - 1;
     float k[8];
     unpack8<T>(reinterpret_cast<const uint4*>(K)[(static_cast<long>(kvh) * max_seq + jr) * L + c],
                k);
-    const int h1 = first_head(kvh + 1, nh, nkv);
-    for (int h = first_head(kvh, nh, nkv); h < h1; ++h) {
+    const int h0 = first_head(kvh, nh, nkv) + blockIdx.z * per;
+    const int end = first_head(kvh + 1, nh, nkv), h1 = h0 + per < end ? h0 + per : end;
+    for (int h = h0; h < h1; ++h) {
         float q[8], acc = 0.0f;
         unpack8<T>(reinterpret_cast<const uint4*>(Q)[static_cast<long>(h) * L + c], q);
 #pragma unroll
@@ -490,6 +493,20 @@ int check_attn(const char* fn, int nh, int nkv, int hd, int max_seq, int seq_len
     return 0;
 }
 
+// A block's q heads go one after the other, so they are spread over blocks (z)
+// until there are 4 blocks per CU.  us, general kernel / all heads in a block /
+// this: 64 heads on 1, head_dim 128, 1 / 200 / 1000 / 8192 positions 2.1 / 12.7 /
+// 2.1, 3.2 / 15.1 / 2.5, 8.3 / 14.6 / 3.2, 52 / 15.6 / 9.2; 8 on 1, 1 / 1000 / 4096
+// 2.0 / 3.0 / 2.1, 2.8 / 3.4 / 2.2, 5.2 / 3.5 / 2.8; 20 on 5, 1 / 200 / 2500 2.1 /
+// 2.6 / 2.2, 2.4 / 2.7 / 2.2, 7.1 / 3.1 / 3.1.
+dim3 scores_rows_grid(int row_blocks, int nh, int nkv, int* per) {
+    const int group = (nh + nkv - 1) / nkv;  // the most q heads of a kv head
+    const long blocks = static_cast<long>(row_blocks) * nkv;
+    const long want = std::min<long>(group, std::max(1L, 4L * device_cu_count() / blocks));
+    *per = static_cast<int>((group + want - 1) / want);
+    return dim3(row_blocks, nkv, (group + *per - 1) / *per);
+}
+
 template <class T>
 int attention_scores(const char* fn, const uint16_t* Q, const uint16_t* K, float* sc, int nh,
                      int nkv, int hd, int max_seq, int seq_len, float scale, spb_stream_t s) {
@@ -499,12 +516,13 @@ int attention_scores(const char* fn, const uint16_t* Q, const uint16_t* K, float
     if (!Q || !K || !sc) return invalid("%s: null pointer", fn);
     if (al16(Q) && al16(K) && (hd == 32 || hd == 64 || hd == 128 || hd == 256)) {
         const int rows = kOpBlock / (hd / 8);
-        const dim3 grid((seq_len + rows - 1) / rows, nkv);
+        int per = 1;
+        const dim3 grid = scores_rows_grid((seq_len + rows - 1) / rows, nh, nkv, &per);
         switch (hd) {
-        case 32: hipLaunchKernelGGL((attention_scores_rows_kernel<T, 4>), grid, dim3(kOpBlock), 0, as_stream(s), Q, K, sc, nh, nkv, max_seq, seq_len, scale); break;
-        case 64: hipLaunchKernelGGL((attention_scores_rows_kernel<T, 8>), grid, dim3(kOpBlock), 0, as_stream(s), Q, K, sc, nh, nkv, max_seq, seq_len, scale); break;
-        case 128: hipLaunchKernelGGL((attention_scores_rows_kernel<T, 16>), grid, dim3(kOpBlock), 0, as_stream(s), Q, K, sc, nh, nkv, max_seq, seq_len, scale); break;
-        default: hipLaunchKernelGGL((attention_scores_rows_kernel<T, 32>), grid, dim3(kOpBlock), 0, as_stream(s), Q, K, sc, nh, nkv, max_seq, seq_len, scale); break;
+        case 32: hipLaunchKernelGGL((attention_scores_rows_kernel<T, 4>), grid, dim3(kOpBlock), 0, as_stream(s), Q, K, sc, nh, nkv, max_seq, seq_len, scale, per); break;
+        case 64: hipLaunchKernelGGL((attention_scores_rows_kernel<T, 8>), grid, dim3(kOpBlock), 0, as_stream(s), Q, K, sc, nh, nkv, max_seq, seq_len, scale, per); break;
+        case 128: hipLaunchKernelGGL((attention_scores_rows_kernel<T, 16>), grid, dim3(kOpBlock), 0, as_stream(s), Q, K, sc, nh, nkv, max_seq, seq_len, scale, per); break;
+        default: hipLaunchKernelGGL((attention_scores_rows_kernel<T, 32>), grid, dim3(kOpBlock), 0, as_stream(s), Q, K, sc, nh, nkv, max_seq, seq_len, scale, per); break;
         }
         return launch_status(fn);
     }

@@ -1,5 +1,6 @@
 // Which kernel a call launches, by its grid, under the fake runtime of
-// fake_hip.hpp (256 CUs): the lines between the tiles of the sparse GEMMs.
+// fake_hip.hpp (256 CUs): the lines between the tiles of the sparse GEMMs, and the
+// heads of a block of the per-op attention scores.
 // Prints one line per check and returns the number of failed ones.
 #include <cstdio>
 #include <vector>
@@ -36,6 +37,20 @@ void sparse_i8(int m, int k, int n, int tile_rows, int tile_tokens) {
     check("int8", spb_sparse_i8_gemm(g_words, g_x, g_y, m, k, n, nullptr), m, k, n, tile_rows,
           tile_tokens);
 }
+
+// Scores with the grid of 16 positions (head_dim 128) x kv heads x parts of a group.
+void scores(int nh, int nkv, int seq, int parts) {
+    const uint16_t* w = reinterpret_cast<const uint16_t*>(g_words);
+    float* f = reinterpret_cast<float*>(g_words);
+    g_launches = 0;
+    const int rc = spb_attention_scores_f16(w, w, f, nh, nkv, 128, 8192, seq, 1.0f, nullptr);
+    const dim3 s = g_grid;
+    const bool ok = rc == 0 && g_launches == 1 && static_cast<int>(s.x) == (seq + 15) / 16 &&
+                    static_cast<int>(s.y) == nkv && static_cast<int>(s.z) == parts;
+    std::printf("%s scores %d on %d, %d positions: %u x %u x %u\n", ok ? "ok  " : "FAIL", nh, nkv,
+                seq, s.x, s.y, s.z);
+    g_bad += !ok;
+}
 }  // namespace
 
 int main() {
@@ -61,5 +76,12 @@ int main() {
     sparse_i8(40960, 2560, 33, 256, 128);
     sparse_i8(6912, 2560, 768, 256, 128);
     sparse_i8(6912, 2560, 640, 96, 32);
+    // heads of a group over blocks until there are 4 per CU
+    scores(64, 1, 1, 64);
+    scores(64, 1, 1000, 16);
+    scores(8, 1, 1, 8);
+    scores(8, 1, 8192, 2);
+    scores(20, 5, 513, 4);
+    scores(20, 5, 2500, 1);
     return g_bad;
 }
