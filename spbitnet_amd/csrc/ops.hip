@@ -539,9 +539,25 @@ int attention_output(const char* fn, const float* sc, const uint16_t* V, uint16_
     if (int e = check_attn(fn, nh, nkv, hd, max_seq, seq_len)) return e;
     if (hd > 256) return invalid("%s: head_dim %d > 256", fn, hd);
     if (!sc || !V || !out) return invalid("%s: null pointer", fn);
-    if (al16(V) && hd % 8 == 0) {
+    // A few positions are one round trip and short sums, which the general
+    // kernel's four waves per head finish first.  us, general -> 8 dims per
+    // block: 20 heads on 5, head_dim 128, 1 / 8 / 16 / 32 positions 2.2 -> 2.7, 2.4
+    // -> 2.7, 2.8 -> 2.7, 3.8 -> 2.7; 64 on 64, 256, 1 / 16 / 32 2.3 -> 4.7, 3.6 ->
+    // 4.7, 5.1 -> 4.6; 8 on 1, 64, 8 / 16 2.2 -> 2.4, 2.4 -> 2.3.
+    if (al16(V) && hd % 8 == 0 && seq_len > std::min(8 + nh / 4, 24)) {
         const int group = (nh + nkv - 1) / nkv;  // the most q heads of a kv head
-        const int per = group >= 4 ? 4 : (group >= 2 ? 2 : 1);
+        // Up to a position per thread a block's time is its sums over the
+        // threads, 8 for every head: one head, or as many as leave 2 blocks per
+        // CU.  us with 1 / 2 / 4, 64 positions: 20 on 5, head_dim 128 2.7 / 2.7 /
+        // 3.1; 64 on 1, 64 2.8 / 2.7 / 3.2, 128 3.3 / 3.1 / 3.2, 256 4.6 / 3.9 /
+        // 3.9.  Past that, the reads of V that heads share (2500 positions: 20
+        // on 5, 128 6.4 / 5.0 / 5.3, 256 21.4 / 13.3 / 11.4).
+        int per = group >= 4 ? 4 : (group >= 2 ? 2 : 1);
+        if (seq_len <= kOutBlock)
+            for (int p = 1; p < per; p *= 2)
+                if (static_cast<long>(hd / 8) * nkv * ((group + p - 1) / p) <=
+                    2L * device_cu_count())
+                    per = p;
         const dim3 grid(hd / 8, nkv, (group + per - 1) / per), block(kOutBlock);
         switch (per) {
         case 1: hipLaunchKernelGGL((attention_output_cols_kernel<T, 1>), grid, block, 0, as_stream(s), sc, V, out, nh, nkv, hd, max_seq, seq_len); break;

@@ -1,6 +1,6 @@
 // Which kernel a call launches, by its grid, under the fake runtime of
-// fake_hip.hpp (256 CUs): the lines between the tiles of the sparse GEMMs, and the
-// heads of a block of the per-op attention scores.
+// fake_hip.hpp (256 CUs): the lines between the tiles of the sparse GEMMs and
+// between the forms of the per-op attention.
 // Prints one line per check and returns the number of failed ones.
 #include <cstdio>
 #include <vector>
@@ -38,17 +38,25 @@ void sparse_i8(int m, int k, int n, int tile_rows, int tile_tokens) {
           tile_tokens);
 }
 
-// Scores with the grid of 16 positions (head_dim 128) x kv heads x parts of a group.
-void scores(int nh, int nkv, int seq, int parts) {
+// Scores with the grid of 16 positions (head_dim 128) x kv heads x parts of a
+// group, outputs with that of head_dim 128 / 8 x kv heads x parts of a group, or
+// of one block per head (parts 0).
+void attention(int nh, int nkv, int seq, int score_parts, int output_parts) {
     const uint16_t* w = reinterpret_cast<const uint16_t*>(g_words);
     float* f = reinterpret_cast<float*>(g_words);
     g_launches = 0;
-    const int rc = spb_attention_scores_f16(w, w, f, nh, nkv, 128, 8192, seq, 1.0f, nullptr);
+    const int r0 = spb_attention_scores_f16(w, w, f, nh, nkv, 128, 8192, seq, 1.0f, nullptr);
     const dim3 s = g_grid;
-    const bool ok = rc == 0 && g_launches == 1 && static_cast<int>(s.x) == (seq + 15) / 16 &&
-                    static_cast<int>(s.y) == nkv && static_cast<int>(s.z) == parts;
-    std::printf("%s scores %d on %d, %d positions: %u x %u x %u\n", ok ? "ok  " : "FAIL", nh, nkv,
-                seq, s.x, s.y, s.z);
+    const int r1 = spb_attention_output_f16(f, w, reinterpret_cast<uint16_t*>(g_words), nh, nkv,
+                                            128, 8192, seq, nullptr);
+    const dim3 o = g_grid;
+    const dim3 os = output_parts ? dim3(16, nkv, output_parts) : dim3(nh);
+    const bool ok = r0 == 0 && r1 == 0 && g_launches == 2 &&
+                    static_cast<int>(s.x) == (seq + 15) / 16 && static_cast<int>(s.y) == nkv &&
+                    static_cast<int>(s.z) == score_parts && o.x == os.x && o.y == os.y &&
+                    o.z == os.z;
+    std::printf("%s attention %d on %d, %d positions: scores %u x %u x %u, output %u x %u x %u\n",
+                ok ? "ok  " : "FAIL", nh, nkv, seq, s.x, s.y, s.z, o.x, o.y, o.z);
     g_bad += !ok;
 }
 }  // namespace
@@ -77,11 +85,16 @@ int main() {
     sparse_i8(6912, 2560, 768, 256, 128);
     sparse_i8(6912, 2560, 640, 96, 32);
     // heads of a group over blocks until there are 4 per CU
-    scores(64, 1, 1, 64);
-    scores(64, 1, 1000, 16);
-    scores(8, 1, 1, 8);
-    scores(8, 1, 8192, 2);
-    scores(20, 5, 513, 4);
-    scores(20, 5, 2500, 1);
+    attention(64, 1, 1, 64, 0);
+    attention(64, 1, 24, 64, 0);
+    attention(64, 1, 25, 64, 32);
+    attention(64, 1, 1000, 16, 16);
+    attention(8, 1, 1, 8, 0);
+    attention(8, 1, 11, 8, 8);
+    attention(8, 1, 8192, 2, 2);
+    attention(20, 5, 13, 4, 0);
+    attention(20, 5, 512, 4, 4);
+    attention(20, 5, 513, 4, 1);
+    attention(20, 5, 2500, 1, 1);
     return g_bad;
 }

@@ -16,7 +16,10 @@ pytestmark = pytest.mark.gpu
 SHAPES = [  # heads, kv heads, head_dim, seq
     (4, 2, 32, 1), (20, 5, 128, 63), (8, 1, 64, 511), (7, 3, 128, 513), (16, 16, 64, 1025),
     (3, 1, 256, 2049), (20, 5, 128, 5000), (5, 2, 80, 700), (2, 2, 20, 130), (9, 1, 8, 300),
-    (64, 1, 128, 1300), (8, 1, 64, 4500),  # groups over several blocks
+    # groups over several blocks, the
+    # last lengths of the general output kernel and the first of 1, 2 and 4 heads a block
+    (64, 1, 128, 1300), (8, 1, 64, 4500), (64, 1, 64, 24), (64, 1, 64, 25), (64, 1, 128, 400),
+    (64, 1, 256, 512), (20, 5, 128, 13), (20, 5, 128, 14), (20, 5, 128, 512),
 ]
 
 
