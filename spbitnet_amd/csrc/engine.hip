@@ -62,10 +62,18 @@ int batch_groups(int batch) { return batch >= 24 && batch <= 32 ? 2 : 1; }
 // ... in the step graphs whose attention reaches more than this many splits
 // (768 positions).  Below, the second branch's launches and its second read of
 // the weights cost more than their overlap with the attention gives.  2B
-// shape, us per step, two groups -> one: 32 sequences at positions 100 / 300 /
-// 500 / 750 1710-1854 -> 1663-1673, 1808 -> 1825, 1959 -> 1941, 2010 -> 2031;
-// at 1000 / 2048 2065 -> 2144, 2544 -> 2657; 24 sequences 1842-1942 -> 1603-
-// 1617, 1743 -> 1739, 1843 -> 1814, 1901 -> 1898, 1922 -> 1979, 2287 -> 2394.
+// shape, us per step, two groups -> one, on two boxes (runs of two branches differ by
+// up to 8 %, of one by 1 %):
+//   32 sequences at position 100 1710-1854 -> 1663-1673, 1897-1930 -> 1659-1674;
+//   300 1808 -> 1825, 1828-1846 -> 1791; 500 1959 -> 1941, 1873-1880 -> 1832;
+//   750 2010 -> 2031, 2037-2078 -> 1959; 1000 2065 -> 2144, 2104-2111 -> 2069;
+//   2048 2544 -> 2657, 2554-2566 -> 2605;
+//   24 sequences at 100 1842-1942 -> 1603-1617, 1858-1936 -> 1590; 300 1743 ->
+//   1739, 1830-1876 -> 1720; 500 1843 -> 1814, 1860-1883 -> 1752; 750 1901 -> 1898,
+//   2070-2076 -> 1827; 1000 1922 -> 1979, 2062-2072 -> 1919; 2048 2287 -> 2394,
+//   2271-2287 -> 2316.
+// So below the line one group is never more than 1 % behind, and where past it
+// the second begins to pay differs between the boxes.
 constexpr int kGroupSplits = 12;
 constexpr long kPrefillPartialBytes = (1L << 31) - 1;  // split partials of one pass (at most)
 constexpr int kPrefillMinDefault = 16;   // prompt tokens before the last that switch to it
@@ -1576,9 +1584,8 @@ __global__ __launch_bounds__(kAttnThreads) void attention_kernel(
 // qkv_stride, its partials after those of t - 1; consecutive tokens of one
 // sequence at consecutive positions), on the float32 matrix cores.  v_mfma_f32_16x16x4_f32 adds its four
 // products to the accumulator one after the other (k ascending), each as a
-// fused multiply-add rounded to nearest even, denormals kept: compared bit
-// for bit with fmaf on 21 M sums over normal, wide-exponent and denormal
-// operands.  So a chain of them is attention_split's fma chain, and every
+// fused multiply-add rounded to nearest even, denormals kept
+// (tests/cpp/mfma_chain.hip compares its bits with fmaf's).  So a chain of them is attention_split's fma chain, and every
 // partial equals that of the token's decode step:
 //   score = ((a0 + a1) + (a2 + a3)) * scale, a_w = fma chain over quarter w,
 //   the softmax of split_softmax, and acc = fma over j ascending of e_j v_j.
@@ -1600,9 +1607,9 @@ __global__ __launch_bounds__(kAttnThreads) void attention_kernel(
 // VALU instructions of a SIMD's waves add up (15.2 ns per MFMA, ~1 ns more per
 // VALU instruction, measured).  Hence float32 operands in LDS: unpacking them
 // at each use took 256 more VALU instructions per tile (5.2 against 6.8 us for
-// a tile of a lone wave).  A 2048-token prompt's two passes of the 2B shape:
-// 197 + 375 us per layer with the VALU form this replaces, 74 + 171 us now
-// (5.3 us per tile and SIMD, 3.9 of it MFMA).
+// a tile of a lone wave).  Two passes of 1024 tokens of the 2B shape, us per
+// layer: 197 + 375 with the VALU form this replaces, 74 + 171 with this; one pass
+// of 2047 252 (5.3 us per tile and SIMD, 3.9 of it MFMA).
 __device__ __forceinline__ void swap16(float& a, float& b) {
     const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(a), __float_as_uint(b), false,
                                                     false);
@@ -3126,7 +3133,6 @@ void launch_attention_hd(int G, dim3 grid, hipStream_t s, const uint16_t* qkv,
         break;
     }
 }
-// The prefill form: c tokens at positions pos0 .. pos0 + c - 1 (grid.z).
 // Tokens t0 .. t0 + n - 1 of a prefill pass: sequence seq's positions pos0 ..
 // pos0 + n - 1.
 struct PrefillSeg {
@@ -3274,12 +3280,15 @@ void launch_attn_combine(int hd, int nh, int splits, hipStream_t s, const float*
 // itself (the same operations in the same order), a launch and a trip through
 // memory less.  Few: up to 4, and up to 8 where a token's heads are at most
 // kFoldLongCols wide (wider ones have too many loads for one block).  Decode
-// steps of 6 layers, us, apart -> folded: 2560 wide, 2 / 32 / 128 sequences at
+// steps of 6 layers, us, apart -> folded, 2 / 32 / 128 sequences: 2560 wide at
 // position 60 313 -> 304, 378 -> 368, 570 -> 557, at 450 317 -> 316, 427 -> 423,
-// 697 -> 692; 4096 wide at 200 394 -> 387, 522 -> 513, 765 -> 755, at 300 395 ->
-// 401, 548 -> 556, 836 -> 844.  Prompts through 4 layers: 4096 wide, 200 / 300 /
-// 500 tokens 656 -> 649, 767 -> 774, 936 -> 950; 8192 wide, 200 / 400 / 500 941 ->
-// 934, 1341 -> 1360, 1519 -> 1543.
+// 697 -> 692; 3072 wide at 300 351 -> 351, 493 -> 489, 725 -> 720, at 450 352 ->
+// 353, 505 -> 509, 778 -> 767; 3584 wide at 300 368 -> 370, 529 -> 529, 797 -> 793;
+// 4096 wide at 200 394 -> 387, 522 -> 513, 765 -> 755, at 300 395 -> 401, 548 ->
+// 556, 836 -> 844.  Prompts through 4 layers, 200 / 300 / 500 tokens: 3072 wide 592
+// -> 583, 674 -> 676, 801 -> 803; 3584 614 -> 605, 722 -> 725, 858 -> 863; 4096 656
+// -> 649, 767 -> 774, 936 -> 950; 8192 wide, 200 / 400 / 500 941 -> 934, 1341 ->
+// 1360, 1519 -> 1543.
 constexpr int kFoldLongCols = 3072;
 void launch_attn_input(int hd, int nh, int splits, hipStream_t s, const float* pm,
                        const float* pl, const float* pacc, float* comb, const EngineState* st,
@@ -3374,11 +3383,13 @@ hipError_t gemm_group(const spb_sparse_linear* const* w, int nw, const int8_t* X
 }
 
 // Sinks fused into the GEMM at every batch size; the q/k/v sink only up to
-// kFuseTokens tokens: in a 1024-token prefill pass its epilogue (decode
-// state and RoPE row loads per lane, pair stores to the KV cache) made the
-// GEMM longer than GEMM + sink kernel (33.8 against 20.7 + 10.1 us), while
-// the bf16 and residual sinks gained (gate|up 69.4 against 61.1 + 28.0 us,
-// down 40.1 against 36.3 + 7.6 us).
+// kFuseTokens tokens: its epilogue (decode state and RoPE row loads per lane,
+// pair stores to the KV cache) makes the GEMM longer than the sink kernel costs.
+// Prompts through 10 layers of the 2B shape, us, apart -> fused: 33 / 64 tokens
+// 1173 -> 1165, 1209 -> 1205; 96 / 199 / 512 / 1024 / 1499 / 2048 1340 -> 1368, 1420
+// -> 1438, 2007 -> 2043, 3067 -> 3080, 4412 -> 4460, 6712 -> 6704.  The bf16 and
+// residual sinks gain everywhere (1024 tokens: gate|up 69.4 against 61.1 + 28.0
+// us, down 40.1 against 36.3 + 7.6 us).
 template <class Sink>
 struct SinkFusesWide {
     static constexpr bool value = true;

@@ -16,13 +16,16 @@
 //     one step; the four lane groups hold four steps, and exchanging them
 //     (transpose) gives every lane its own words of four steps.
 //   * Activations go from memory to LDS without passing registers.
-// What bounds it (cycle counts around the parts of a step, one block on a CU):
-// ~600 cycles per wave of decode (54 VALU instructions, 5 cycles each and two
-// waves per SIMD), ~500 of addresses, exchanges and load issue, ~630 of operand
-// reads and 16 SMFMACs (18 cycles each), ~100 of waiting for loads; SMFMACs and
-// VALU instructions of different waves overlap only in part (7.5 ns per SMFMAC,
-// 1.0-1.3 ns more per VALU instruction in its shadow).  Interleaving them by
-// hand, 128 x 64 tiles per wave and 256 tokens per block ran at the same speed.
+// What bounds it: the length of a step, and the CU with the most blocks.  13824 x
+// 2560, n = 2048 (864 blocks, 87 us): the matrix units are busy 17 % of the time,
+// the LDS 20 % (no conflicts), the VALU 24 %; a wave spends 41 % of its life
+// waiting for loads, LDS or the barrier and 44 % waiting to issue.  The
+// decode does not hold it: the int8 operand, which needs none (VALU 8 %), takes
+// the same 85-88 us.  20 steps take 32 us with a block on a CU and 46 with two
+// (256 and 512 blocks), then 70, 84 and 108-120 us with a third, fourth and fifth
+// on some CU (528 to 768, 864 to 1024 and 1026 to 1040 blocks), so a grid pays
+// for whole blocks per CU.  Interleaving VALU and SMFMACs by hand, 128 x 64 tiles
+// per wave and 256 tokens per block ran at the same speed.
 #pragma once
 
 #include "smfmac.hpp"
@@ -88,9 +91,9 @@ struct WideTernary {
     struct Held {
         uint32_t m[kWideOwn][4], v[kWideOwn][4];
     };
-    // Steps step0 .. step0 + 3 of strips strip0 .. strip0 + 3.  Rows past the
-    // matrix read its last row and steps past the row its last step; neither
-    // feeds a stored result.
+    // Steps step0 .. step0 + 3 of strips strip0 .. strip0 + kWideOwn - 1.  Rows
+    // past the matrix read its last row and steps past the row its last step;
+    // neither feeds a stored result.
     __device__ void load(Raw& r, int strip0, int step0, int nsteps, int lane) const {
         const int st = min(step0 + (lane >> 4), nsteps - 1);
 #pragma unroll
@@ -250,7 +253,7 @@ __global__ __launch_bounds__(kWideThreads, 4) void gemm_wide_kernel(A src,
     if (s < nsteps) step(s, 0);  // uniform
     if (s + 1 < nsteps) step(s + 1, 1);
     if (s + 2 < nsteps) step(s + 2, 2);
-    // lane (li, q) of tile (s, t) holds rows 16 (8 ws + s) + 4q .. + 3 of token 16 (4 wt + t) + li
+    // lane (li, q) of tile (e, t) holds rows 16 (4 ws + e) + 4 q .. + 3 of token 16 (4 wt + t) + li
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
         const int row = r0 + 16 * (4 * ws + e) + 4 * q;
