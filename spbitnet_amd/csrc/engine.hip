@@ -62,7 +62,7 @@ int batch_groups(int batch) { return batch >= 24 && batch <= 32 ? 2 : 1; }
 // ... in the step graphs whose attention reaches more than this many splits
 // (768 positions).  Below, the second branch's launches and its second read of
 // the weights cost more than their overlap with the attention gives.  2B
-// shape, us per step, two groups -> one, on two boxes (runs of two branches differ by
+// shape, us per step, two groups -> one, on two machines (runs of two branches differ by
 // up to 8 %, of one by 1 %):
 //   32 sequences at position 100 1710-1854 -> 1663-1673, 1897-1930 -> 1659-1674;
 //   300 1808 -> 1825, 1828-1846 -> 1791; 500 1959 -> 1941, 1873-1880 -> 1832;
@@ -73,7 +73,7 @@ int batch_groups(int batch) { return batch >= 24 && batch <= 32 ? 2 : 1; }
 //   2070-2076 -> 1827; 1000 1922 -> 1979, 2062-2072 -> 1919; 2048 2287 -> 2394,
 //   2271-2287 -> 2316.
 // So below the line one group is never more than 1 % behind, and where past it
-// the second begins to pay differs between the boxes.
+// the second begins to pay differs between the machines.
 constexpr int kGroupSplits = 12;
 constexpr long kPrefillPartialBytes = (1L << 31) - 1;  // split partials of one pass (at most)
 constexpr int kPrefillMinDefault = 16;   // prompt tokens before the last that switch to it
