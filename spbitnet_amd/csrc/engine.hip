@@ -3811,6 +3811,7 @@ extern "C" int spb_engine_create(const spb_model_config* cfg, const spb_transfor
                                  const uint16_t* embed_tokens, const uint16_t* lm_head,
                                  const float* final_norm, int max_seq, spb_engine** out) {
     clear_error();
+    (void)hipGetLastError();  // not ours: the checks below take it for a launch's
     const char* fn = "spb_engine_create";
     if (!cfg || !layers || !embed_tokens || !final_norm || !out)
         return invalid("%s: null argument", fn);
@@ -3984,6 +3985,7 @@ extern "C" int spb_engine_forward(spb_engine* e, int token_id, const float** d_l
 extern "C" int spb_engine_generate(spb_engine* e, const int* prompt, int n_prompt, int n_new,
                                    int stop_at_eos, int* out_tokens, int* n_generated) {
     clear_error();
+    (void)hipGetLastError();  // not ours: the checks below take it for a launch's
     const char* fn = "spb_engine_generate";
     if (!e || !prompt || (!out_tokens && n_new > 0)) return invalid("%s: null argument", fn);
     if (n_prompt <= 0 || n_new < 0) return invalid("%s: need n_prompt >= 1, n_new >= 0", fn);
@@ -4367,6 +4369,7 @@ extern "C" int spb_batch_engine_create(const spb_model_config* cfg,
                                        const float* final_norm, int max_seq, int batch,
                                        spb_batch_engine** out) {
     clear_error();
+    (void)hipGetLastError();  // not ours: the checks below take it for a launch's
     const char* fn = "spb_batch_engine_create";
     if (!cfg || !layers || !embed_tokens || !final_norm || !out)
         return invalid("%s: null argument", fn);
@@ -4543,6 +4546,7 @@ extern "C" int spb_batch_engine_generate(spb_batch_engine* e, const int* prompts
                                          const int* prompt_lens, int n_seq, int n_new,
                                          int stop_at_eos, int* out_tokens, int* n_generated) {
     clear_error();
+    (void)hipGetLastError();  // not ours: the checks below take it for a launch's
     const char* fn = "spb_batch_engine_generate";
     if (!e || !prompts || !prompt_lens || (!out_tokens && n_new > 0))
         return invalid("%s: null argument", fn);

@@ -113,7 +113,11 @@ void launches() {
                                                std::to_string(silent) + " of " +
                                                std::to_string(creating) + " returned 0");
         arm(-1);
-        check(e.generate(lens) == 0, kind + ": generate afterwards");
+        g_pending = hipErrorNotReady;
+        check(e.generate(lens) == 0, kind + ": generate afterwards, an earlier call's error pending");
+        g_pending = hipErrorNotReady;
+        Engine f;
+        check(f.create(s, 4096, batch) == 0, kind + ": create with an earlier call's error pending");
     }
 }
 
